@@ -67,6 +67,7 @@ CAPI_SOURCES = [
     "fft2d.hip",
     "pruned.hip",
     "ns.hip",
+    "ns_grid.hip",
     "registry.cpp",
     "capi.cpp",
 ]

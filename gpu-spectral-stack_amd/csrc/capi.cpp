@@ -356,6 +356,23 @@ int spx_ns_steps(const void* w_in, void* w_out, void* work, const void* forcing_
     });
 }
 
+int spx_ns_grid_supports(int n) { return spx::ns_grid_supports(n) ? 1 : 0; }
+
+int spx_ns_grid_workspace(int n, int pruned, int batch, size_t* count)
+{
+    return guarded([&] { *count = spx::ns_grid_workspace(n, pruned != 0, batch); });
+}
+
+int spx_ns_grid_steps(const void* w_in, void* w_out, void* work, const void* forcing_hat,
+                      const float* nu, int nu_stride, float drag, float dt, int n, int pruned,
+                      int batch, int steps, hipStream_t stream)
+{
+    return guarded([&] {
+        spx::ns_grid_steps(cc(w_in), cm(w_out), cm(work), cc(forcing_hat), nu, nu_stride, drag,
+                           dt, n, pruned != 0, batch, steps, stream);
+    });
+}
+
 int spx_rf_max_nfft(int impl)
 {
     if (impl < 0 || impl >= spx::impl_count() || spx::impls()[impl].rf == nullptr) {

@@ -235,6 +235,11 @@ void scatter_modes(const cf32* modes, cf32* full, int n1, int w, int m1, int m2,
 // --- the Navier-Stokes caller (ns.hip): one fused IMEX stage per field ----------------------
 // Modes in the FNO layout with m = n/3 + 1 ((2m) x m per field). stage 0: out_f = F(state),
 // out_w = the predictor; stage 1: out_w = the corrector from w0, f0 and F(state).
+bool ns_grid_supports(int n);
+std::size_t ns_grid_workspace(int n, bool pruned, int batch);
+void ns_grid_steps(const cf32* w_in, cf32* w_out, cf32* work, const cf32* forcing_hat,
+                   const float* nu, int nu_stride, float drag, float dt, int n, bool pruned,
+                   int batch, int steps, hipStream_t stream);
 bool ns_supports(int n);
 void ns_stage(const cf32* state, const cf32* w0, const cf32* f0, cf32* out_f, cf32* out_w,
               const cf32* forcing_hat, const float* nu, int nu_stride, float drag, float dt,

@@ -566,6 +566,45 @@ at::Tensor ns_advance_op(const at::Tensor& w_hat, const at::Tensor& forcing_hat,
     return out;
 }
 
+// `steps` >= 1 whole steps on a grid without a one-workgroup kernel, or of the rfft2 layout.
+at::Tensor ns_advance_grid_op(const at::Tensor& w_hat, const at::Tensor& forcing_hat,
+                              const at::Tensor& nu, double drag, double dt, int64_t n,
+                              int64_t steps, bool pruned)
+{
+    check_complex64_cuda(w_hat, "w_hat");
+    check_complex64_cuda(forcing_hat, "forcing_hat");
+    TORCH_CHECK(n >= 1 && n <= INT_MAX && spx_ns_grid_supports(static_cast<int>(n)) == 1,
+                "ns_advance_grid: supports n = 32 to 1024, a power of two, got ", n);
+    const int64_t rows = pruned ? 2 * (n / 3 + 1) : n;
+    const int64_t cols = pruned ? n / 3 + 1 : n / 2 + 1;
+    TORCH_CHECK(w_hat.dim() >= 2 && w_hat.size(-2) == rows && w_hat.size(-1) == cols,
+                "ns_advance_grid: w_hat must hold (..., ", rows, ", ", cols, ") modes for n = ", n);
+    TORCH_CHECK(forcing_hat.numel() == rows * cols, "ns_advance_grid: forcing_hat must hold ",
+                rows, " x ", cols, " modes");
+    TORCH_CHECK(nu.is_cuda() && nu.scalar_type() == at::kFloat,
+                "ns_advance_grid: nu must be a float32 CUDA tensor");
+    TORCH_CHECK(steps >= 1 && steps <= INT_MAX, "ns_advance_grid: steps must be >= 1, got ", steps);
+    const int batch = batch_of(w_hat, rows * cols, "ns_advance_grid");
+    TORCH_CHECK(nu.numel() == 1 || nu.numel() == batch,
+                "ns_advance_grid: nu must hold one viscosity or one per field");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(w_hat.device());
+    const at::Tensor w = w_hat.contiguous();
+    const at::Tensor fh = forcing_hat.contiguous();
+    const at::Tensor nc = nu.contiguous();
+    at::Tensor out = at::empty_like(w);
+    if (batch > 0) {
+        size_t count = 0;
+        check_status(spx_ns_grid_workspace(static_cast<int>(n), pruned ? 1 : 0, batch, &count));
+        at::Tensor work = workspace(count, w);
+        check_status(spx_ns_grid_steps(cptr(w), mptr(out), work_ptr(work), cptr(fh),
+                                       nc.const_data_ptr<float>(), nc.numel() == 1 ? 0 : 1,
+                                       static_cast<float>(drag), static_cast<float>(dt),
+                                       static_cast<int>(n), pruned ? 1 : 0, batch,
+                                       static_cast<int>(steps), current_stream()));
+    }
+    return out;
+}
+
 // spectral._C.fft_impls(): the registry's names, in order, as a tuple of str.
 PyObject* py_fft_impls(PyObject*, PyObject*)
 {
@@ -595,10 +634,23 @@ PyObject* py_ns_supports(PyObject*, PyObject* arg)
     return PyBool_FromLong(n > 0 && n < (1L << 30) && spx_ns_supports(static_cast<int>(n)) == 1);
 }
 
+// spectral._C.ns_grid_supports(n): whether ns_advance_grid takes an n x n grid.
+PyObject* py_ns_grid_supports(PyObject*, PyObject* arg)
+{
+    const long n = PyLong_AsLong(arg);
+    if (n == -1 && PyErr_Occurred() != nullptr) {
+        return nullptr;
+    }
+    return PyBool_FromLong(n > 0 && n < (1L << 30)
+                           && spx_ns_grid_supports(static_cast<int>(n)) == 1);
+}
+
 PyMethodDef module_methods[] = {
     {"fft_impls", py_fft_impls, METH_NOARGS, "Names of the FFT implementations, in order."},
     {"ns_supports", py_ns_supports, METH_O,
      "Whether the fused Navier-Stokes stage has a kernel for an n x n grid."},
+    {"ns_grid_supports", py_ns_grid_supports, METH_O,
+     "Whether ns_advance_grid takes an n x n grid."},
     {nullptr, nullptr, 0, nullptr},
 };
 
@@ -629,6 +681,8 @@ TORCH_LIBRARY(spectral, m)
           " float drag, float dt, int n) -> Tensor");
     m.def("ns_advance(Tensor w_hat, Tensor forcing_hat, Tensor nu, float drag, float dt, int n,"
           " int steps) -> Tensor");
+    m.def("ns_advance_grid(Tensor w_hat, Tensor forcing_hat, Tensor nu, float drag, float dt,"
+          " int n, int steps, bool pruned) -> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(spectral, CUDA, m)
@@ -649,6 +703,7 @@ TORCH_LIBRARY_IMPL(spectral, CUDA, m)
     m.impl("ns_predict", &ns_predict_op);
     m.impl("ns_correct", &ns_correct_op);
     m.impl("ns_advance", &ns_advance_op);
+    m.impl("ns_advance_grid", &ns_advance_grid_op);
 }
 
 // Importing spectral._C runs the TORCH_LIBRARY blocks (registering torch.ops.spectral) and

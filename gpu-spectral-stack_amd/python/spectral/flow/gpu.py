@@ -22,6 +22,12 @@ one launch (torch.ops.spectral.ns_advance with one step); advance(w, k), which f
 simulate() use between frames, runs k steps as one launch. The single stages are also exposed
 (torch.ops.spectral.ns_predict / ns_correct). fused=None uses it wherever it applies, True
 requires it, False never.
+
+Where it does not apply (other grids from 32 to 1024, and the full layout) and fused is None, a
+Stockham fft_impl's step() and advance() run each stage as three kernels
+(torch.ops.spectral.ns_advance_grid): inverse columns of the derived fields, rows with the product,
+forward columns with the update. fused=False keeps the transforms and elementwise operations
+apart.
 """
 
 from __future__ import annotations
@@ -130,6 +136,13 @@ class GpuSolver:
                 f"(got pruned={pruned}, fft_impl='{fft_impl}', n={n})"
             )
         self.fused = fusable if fused is None else bool(fused)
+        # step() and advance() by the three-kernel stages, unless fused=False asks for the composed
+        # transforms, drag or dt broadcasts, or a subclass brings its own step.
+        self._grid_steps = (fused is None and not fusable and fft_impl.startswith("stockham")
+                            and _C.ns_grid_supports(n)
+                            and isinstance(flow.drag, (int, float)) and isinstance(dt, (int, float))
+                            and type(self).step is GpuSolver.step
+                            and type(self).tendency is GpuSolver.tendency)
 
         k2 = s.kx**2 + s.ky**2
         over_k2 = torch.where(k2 > 0, 1.0 / k2.clamp(min=1.0), torch.zeros_like(k2))
@@ -166,7 +179,7 @@ class GpuSolver:
         return self.forcing_hat - self.spectral.forward(product) * self.spectral.mask
 
     def step(self, w_hat: torch.Tensor) -> torch.Tensor:
-        if self.fused:
+        if self.fused or self._takes_grid_steps(w_hat):
             return self.advance(w_hat, 1)
         carried = self.explicit * w_hat
         f0 = self.tendency(w_hat)
@@ -184,9 +197,25 @@ class GpuSolver:
             return torch.ops.spectral.ns_advance.default(
                 w_hat, self.forcing_hat, self.nu, float(self.flow.drag), float(self.dt), self.n,
                 steps)
+        if steps > 0 and self._takes_grid_steps(w_hat):
+            return torch.ops.spectral.ns_advance_grid.default(
+                w_hat, self.forcing_hat, self.nu, float(self.flow.drag), float(self.dt), self.n,
+                steps, self.spectral.pruned)
         for _ in range(steps):
             w_hat = self.step(w_hat)
         return w_hat
+
+    def _takes_grid_steps(self, w_hat: torch.Tensor) -> bool:
+        """Whether the three-kernel stages give what the composed step gives for this state: a
+        complex64 state of this layout on the solver's device that needs no gradient, with one
+        viscosity or one per field of exactly its batch shape (others broadcast)."""
+        if not self._grid_steps:
+            return False
+        nu_shape, lead = self.explicit.shape[:-2], w_hat.shape[:-2]
+        return (w_hat.dtype == torch.complex64 and w_hat.device == self.nu.device
+                and w_hat.numel() > 0 and w_hat.shape[-2:] == self.forcing_hat.shape
+                and (nu_shape == lead or (self.nu.numel() == 1 and len(nu_shape) <= len(lead)))
+                and not (w_hat.requires_grad and torch.is_grad_enabled()))
 
     def frames(self, w0: torch.Tensor, steps: int, record_every: int = 1) -> Iterator[torch.Tensor]:
         """Physical vorticity at step 0 (the dealiased initial condition) and after every

@@ -238,3 +238,68 @@ def test_frames_take_the_many_step_path(rng):
         expected.append(solver.to_physical(w_hat))
     for got, want in zip(frames, expected):
         assert torch.equal(got, want)
+
+
+# The three-kernel stages (torch.ops.spectral.ns_advance_grid, C ABI spx_ns_grid_steps), which step()
+# and advance() take on grids and layouts without a one-workgroup kernel: against the composed step.
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pruned", [True, False], ids=["pruned", "full"])
+@pytest.mark.parametrize("n, batch", [(32, 33), (64, 5), (128, 3), (256, 7), (512, 2), (1024, 9)])
+def test_grid_steps_match_the_composed_step(rng, n, batch, pruned):
+    # Odd counts of fields leave partial workgroups; nine fields of 1024^2 run as two groups. The
+    # second state fills every mode of the layout, masked and non-Hermitian ones too. Two float32
+    # orders of the same sums: each is 3e-7 to 5e-7 off 64 bits here.
+    flow, dt = Flow(viscosity=rng.uniform(1e-3, 5e-3, batch), drag=0.1), 1e-3
+    grid = GpuSolver(n, flow, dt, pruned=pruned)
+    if grid.fused:  # these sizes have the one-workgroup kernel; ask the operator itself
+        advance = lambda w, k: torch.ops.spectral.ns_advance_grid(  # noqa: E731
+            w, grid.forcing_hat, grid.nu, 0.1, dt, n, k, pruned)
+    else:
+        advance = grid.advance
+    composed = GpuSolver(n, flow, dt, pruned=pruned, fused=False)
+    smooth = random_state(rng, n, (batch,), composed)
+    every = torch.view_as_complex(torch.as_tensor(
+        rng.standard_normal((*smooth.shape, 2)), dtype=torch.float32, device="cuda"))
+    for w in (smooth, every):
+        kept, expected = w.clone(), w
+        for steps in (1, 2, 3):
+            expected = composed.step(expected)
+            assert relative(advance(w, steps), expected) < 3e-6, f"{steps} steps"
+        assert torch.equal(w, kept)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pruned", [True, False], ids=["pruned", "full"])
+def test_grid_steps_follow_the_float64_solver(rng, pruned):
+    n, steps, dt = 256, 40, 2.5e-3
+    nus = np.array([1e-3, 4e-3])
+    w0 = ref.smooth_random_field(rng, n, batch=(2,))
+    solver = GpuSolver(n, Flow(viscosity=nus, drag=0.1), dt, pruned=pruned)
+    assert solver._grid_steps and not solver.fused
+    gpu = solver.simulate(torch.as_tensor(w0, dtype=torch.float32, device="cuda"), steps, steps)
+    cpu = ref.simulate(w0, nus, 0.1, 1.0, 4, dt, steps, record_every=steps)
+    assert relative(gpu[-1].double(), cpu[-1]) < 1e-5
+
+
+@pytest.mark.gpu
+def test_grid_steps_leave_other_states_to_the_composed_step(rng):
+    n, dt = 32, 1e-3
+    shared = GpuSolver(n, Flow(viscosity=2e-3), dt)
+    per_field = GpuSolver(n, Flow(viscosity=np.array([1e-3, 2e-3, 3e-3])), dt)
+    w = random_state(rng, n, (2, 3), shared)
+    assert shared._takes_grid_steps(w) and shared._takes_grid_steps(w.transpose(0, 1))
+    assert relative(shared.step(w.transpose(0, 1)), shared.step(w).transpose(0, 1)) == 0
+    assert not per_field._takes_grid_steps(w)  # three viscosities broadcast over two rows
+    assert per_field.step(w).shape == w.shape
+    assert not shared._takes_grid_steps(w[:0]) and shared.step(w[:0]).shape == w[:0].shape
+    assert not shared._takes_grid_steps(w.clone().requires_grad_())
+    assert shared.advance(w, 0) is w
+    assert not GpuSolver(n, Flow(), dt, fft_impl="naive")._takes_grid_steps(w)
+    with pytest.raises(RuntimeError, match="w_hat must hold"):
+        torch.ops.spectral.ns_advance_grid(w, shared.forcing_hat, shared.nu, 0.1, dt, n, 1, True)
+    with pytest.raises(RuntimeError, match="32 to 1024"):
+        torch.ops.spectral.ns_advance_grid(w, shared.forcing_hat, shared.nu, 0.1, dt, 16, 1, True)
+    with pytest.raises(RuntimeError, match="steps must be >= 1"):
+        torch.ops.spectral.ns_advance_grid(w, shared.forcing_hat, shared.nu, 0.1, dt, n, 0, False)
