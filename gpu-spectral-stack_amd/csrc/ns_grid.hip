@@ -26,6 +26,11 @@
 // Every pass moves its arrays once; the derived spectra (4 n pitch values per field) are the one
 // large intermediate. Normalization: inverse 1 / n^2, forward none, as numpy. The imaginary parts
 // of a row's zero and n/2 frequencies are dropped, as numpy's irfft drops them.
+//
+// Measured on MI355X (256^2 pruned, 48 fields): columns 12.8 us (38 MB written), rows 13.0 us
+// (38 MB read, 8 MB written), update 10.3 us; a stage was about 105 us composed. About 4 us of
+// each launch is its ramp and drain; neither fewer stages (radix 16) nor the update's loads issued
+// ahead of its transform moved the rest.
 
 #include "stockham.hpp"
 
@@ -56,7 +61,9 @@ struct NsGrid {
     static constexpr int kPitch = (kW + 15) / 16 * 16;     // of P and Q rows: whole 128-byte lines
     static constexpr int kT = N <= 512 ? 16 : 8;           // columns per tile
     static constexpr int kTiles = (kW + kT - 1) / kT;
-    static constexpr int kR = N >= 128 ? 16 : 8;           // radix and values per lane, columns
+    // Radix and values per lane of the columns: 8 while a tile then takes at most 512 lanes. At 256
+    // the update waits on its loads, not on its stages: 12.4 us with 16 values, 10.3 us with 8.
+    static constexpr int kR = N <= 256 ? 8 : 16;
     using PC = ColumnPlan<N, kR, kR>;
     static constexpr int kColumnThreads = kT * PC::L;
     static constexpr int kColumnLds = pad(N - 1) * kT + kT;
@@ -86,6 +93,14 @@ __device__ __forceinline__ float ky_of(int i)
     return static_cast<float>(i < G::N / 2 ? i : i - G::N);
 }
 
+// 1 / x to the last bit or the one before it: the hardware's approximation and one Newton step
+// (a correctly rounded division is four times the instructions).
+__device__ __forceinline__ float reciprocal(float x)
+{
+    const float r = __builtin_amdgcn_rcpf(x);
+    return fmaf(r, fmaf(-x, r, 1.0f), r);
+}
+
 // Multiplier of omega_hat for set 0 .. 3 (P1, Q1 before its conjugation, P2, Q2 likewise):
 //   u + i v: (i ky + kx) / k^2, u - i v: (i ky - kx) / k^2   (u = i ky psi, v = -i kx psi)
 //   wx + i wy: i kx - ky, wx - i wy: i kx + ky
@@ -96,7 +111,7 @@ __device__ __forceinline__ cf32 multiplier(int set, float kx, float ky)
     constexpr float kScale = 1.0f / (static_cast<float>(G::N) * static_cast<float>(G::N));
     if (set < 2) {
         const float k2 = kx * kx + ky * ky;
-        const float f = k2 > 0.0f ? kScale / k2 : 0.0f;
+        const float f = k2 > 0.0f ? kScale * reciprocal(k2) : 0.0f;
         return {(set == 0 ? kx : -kx) * f, ky * f};
     }
     return {(set == 2 ? -ky : ky) * kScale, kx * kScale};
@@ -282,7 +297,7 @@ __global__ void __launch_bounds__(G::kColumnThreads)
             const cf32 F = csub(forcing_hat[at], kept ? v[e] : czero());
             const float linear = -nu_f * (kx * kx + ky * ky) - drag;
             const float ex = 1.0f + 0.5f * dt * linear;
-            const float im = 1.0f / (1.0f - 0.5f * dt * linear);
+            const float im = reciprocal(1.0f - 0.5f * dt * linear);
             const cf32 w = w0[base + at];
             if (stage == 0) {
                 out_f[base + at] = F;
