@@ -10,12 +10,19 @@
 // column tile (N1 rows by TC >= w values): at 128 x 128 with w <= 16, 40 KB, so four arrays share
 // a CU and more of the HBM traffic overlaps the transforms.
 //
-//   forward  every row pass's loads first, then per pass: row transform (exchanges in the
+//   forward  the row passes' loads first, as many passes as fit 32 values per lane, then per pass: row transform (exchanges in the
 //            scratch), bins X[k], k < w, into the tile; the w columns in place down the tile;
 //            the kept rows (0 .. m1-1, n1-m1 .. n1-1) of those columns stored flat.
 //   inverse  the kept modes into the tile (the other rows read as zeros); inverse columns; per
 //            pass: each lane forms its row-inverse inputs straight from the tile row (the c2r
 //            prepare), inverse row transform, the real rows stored.
+//
+// Arrays of 2^15 and 2^16 points (128 x 256, 256 x 128, 256 x 256), whose half spectra fit no
+// workgroup, take the same kernels with 512 or 1024 lanes, in place of a row pass and a column pass
+// through HBM. 256 x 256 x 256, 32 modes, forward / inverse: 28.5 / 29.3 us in two passes, 18.0 /
+// 17.8 us here; 512 arrays 43.7 / 50.1 -> 34.4 / 32.7 us. With one array per compute unit the
+// row transforms' instructions (9 us per array) and the loads at the HBM rate (11 us for 256
+// arrays) overlap pass by pass; the last pass and the columns stay outside.
 //
 // Normalization follows numpy: forward none, inverse 1 / (n1 n2).
 
@@ -23,15 +30,24 @@
 
 namespace spx::dev {
 
-template <int N1_, int M_, int R, bool Table>
+template <int N1_, int M_, int R, bool Table, bool Inv, int WMax_ = M_ / 4>
 struct Modes2d {
     static constexpr int N1 = N1_;  // rows (column transform length)
     static constexpr int M = M_;    // complex values per real row (n2 / 2)
     static constexpr bool kTable = Table;
-    static constexpr int WMax = M / 4;  // kept columns this kernel takes
-    using PR = Plan<M, R, default_e<M, R>()>;
+    static constexpr int WMax = WMax_;  // kept columns this kernel takes
+    // Arrays of 2^15 points and more. Their forward takes 16 values per lane for row transforms of
+    // 128 points (16 x 8 for 8 x 8 x 2), exchanged through half the scratch: a fifth fewer
+    // instructions, which bound the row passes where a compute unit runs one array. 256^2 with 32
+    // columns: 13.1 -> 10.9 us for one array, 18.9 -> 18.1 us for 256. The inverse, which then
+    // stores its shorter runs through the scratch too, was 10 % slower that way.
+    static constexpr bool kLarge = N1 * M > 8192;
+    static constexpr bool kSplit = kRadix16 && R == 8 && M == 128 && kLarge && !Inv;
+    using PR = Plan<M, kSplit ? 16 : R, kSplit ? 16 : default_e<M, R>()>;
     using PC = Plan<N1, column_radix<N1, R>(), column_values<N1, R>()>;  // as Fused2d's
-    static constexpr int NT = 256;
+    // Large arrays: 1024 lanes, or 512 where the tile leaves room for two workgroups per compute
+    // unit.
+    static constexpr int NT = !kLarge ? 256 : N1 * WMax > 4096 ? 1024 : 512;
     static constexpr int RPP = NT / PR::L;        // rows per pass
     static constexpr int kPasses = N1 / RPP;
     // LDS layouts (64 banks of 4 bytes, 8-byte accesses served a half-wave at a time). Scratch
@@ -39,10 +55,13 @@ struct Modes2d {
     // rows of 64 values or more): row f in tile row pad(f), tile rows TC = 4 mod 8 apart. Bank
     // conflicts in the 128 x 128 kernels' row and column passes: 20 % and 14 % of LDS cycles,
     // against 56 % and 50 % with odd strides.
-    static constexpr int TR = M == 64 ? 72 : (pad(M) + 1) | 1;  // scratch row stride
+    // Split scratch rows (floats) sit 136 apart (8 mod 64): conflict-free for 8 lanes of 16.
+    static constexpr int TR = M == 64 ? 72 : kSplit ? 136 : (pad(M) + 1) | 1;  // scratch row stride
     static constexpr bool kPadRows = N1 >= 64 && M >= 64;
     static constexpr int TC = kPadRows ? (WMax + 3) / 8 * 8 + 4 : WMax | 1;  // tile row stride
-    static constexpr int kScratch = RPP * TR;
+    static constexpr int kScratch = kSplit ? RPP * TR / 2 : RPP * TR;  // in complex values
+    // Passes whose row loads are in flight together: 32 values per lane.
+    static constexpr int kAhead = cmin(kPasses, 32 / PR::E);
     static constexpr int kTile = (kPadRows ? pad(N1 - 1) + 1 : N1) * TC;
     using ColLay = std::conditional_t<kPadRows, PaddedRows<TC>, Strided<TC>>;
     __host__ __device__ static constexpr int tile_row(int f)
@@ -52,9 +71,11 @@ struct Modes2d {
     static constexpr int kMaxIo = (N1 * WMax + NT - 1) / NT;  // flat modes per lane, at most
 
     static_assert(kPasses >= 1 && N1 % RPP == 0, "row passes cover the rows exactly");
-    static_assert(kPasses * PR::E <= 32, "every pass's row inputs fit in registers");
+    static_assert(!kSplit || (PR::L == 8 && TR >= pad(M - 1) + 1), "split scratch rows");
     static_assert(PR::L <= 64 && PC::L <= 64, "row and column transforms stay inside a wave");
     static_assert(WMax < PR::L * (WMax / PR::L + 1), "the bin loop covers k < WMax");
+    static_assert((kScratch + kTile) * sizeof(cf32) <= (NT == 512 ? 80 : 160) * 1024,
+                  "LDS: two workgroups of 512 lanes, or one larger");
     static_assert(static_cast<long long>(N1) * WMax * N1 * WMax < (1LL << 31), "FastDiv range");
 
     __device__ __forceinline__ static int row_of(int f, int m1)
@@ -62,6 +83,21 @@ struct Modes2d {
         return f >= m1 ? f + N1 - 2 * m1 : f;
     }
 };
+
+// The row transform of a row held in registers, exchanging in scratch row `prow`.
+template <class F, bool Inv>
+__device__ __forceinline__ void modes_row(cf32 (&v)[F::PR::E], cf32* scratch, int prow, int lane,
+                                          const cf32* table)
+{
+    using PR = typename F::PR;
+    if constexpr (F::kSplit) {
+        float* const s = reinterpret_cast<float*>(scratch) + prow * F::TR;
+        run_stages_split<PR, 0, Inv, F::kTable>(v, s, lane, table);
+    } else {
+        run_stages<PR, 0, Inv, F::kTable, RowExchange<PR, F::TR>>(v, scratch + prow * F::TR, lane,
+                                                                  table);
+    }
+}
 
 // Forward: z = the real arrays viewed as complex (batch x N1 x M), y = batch arrays of 2 m1 x w
 // modes. wdiv divides by w.
@@ -78,24 +114,25 @@ __global__ void __launch_bounds__(F::NT)
     const int tid = threadIdx.x;
     const int lane = tid % PR::L;
     const int prow = tid / PR::L;  // row within a pass
-    cf32* const s = lds + prow * F::TR;
 
-    // Every pass's loads in pass order, so pass p's transform waits for its own loads only.
+    // The loads in pass order, kAhead passes in flight, so pass p's transform waits for its own
+    // loads only.
     constexpr int R0 = PR::template radix<0>();
     const cf32* const src = z + array * F::N1 * F::M;
-    cf32 v[F::kPasses][PR::E];
-    static_for<0, F::kPasses>([&](auto pi) {
+    cf32 v[F::kAhead][PR::E];
+    const auto fetch = [&](auto pi) {
         constexpr int p = decltype(pi)::value;
         const cf32* const row = src + (p * F::RPP + prow) * F::M;
 #pragma unroll
         for (int b = 0; b < PR::E / R0; ++b) {
 #pragma unroll
             for (int r = 0; r < R0; ++r) {
-                v[p][b * R0 + r] = row[input_index<PR, 0>(lane, b, r)];
+                v[p % F::kAhead][b * R0 + r] = row[input_index<PR, 0>(lane, b, r)];
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-    });
+    };
+    static_for<0, F::kAhead>(fetch);
 
     // Rows: transform, then X[k] = E[k] + exp(-pi i k / M) O[k] for k < w into the tile. The
     // lane holds Z[k] for its k = lane + j L; the partner Z[M - k] is element (L - lane) + (E - 1
@@ -109,13 +146,14 @@ __global__ void __launch_bounds__(F::NT)
     const int mirror = (wave_lane & ~(PR::L - 1)) | ((PR::L - lane) & (PR::L - 1));
     static_for<0, F::kPasses>([&](auto pi) {
         constexpr int p = decltype(pi)::value;
-        run_stages<PR, 0, false, F::kTable, RowExchange<PR, F::TR>>(v[p], s, lane, table);
+        cf32(&u)[PR::E] = v[p % F::kAhead];
+        modes_row<F, false>(u, lds, prow, lane, table);
         cf32* const trow = tile + F::tile_row(p * F::RPP + prow);
         static_for<0, (F::WMax + PR::L - 1) / PR::L>([&](auto ji) {
             constexpr int j = decltype(ji)::value;
-            const cf32 zk = v[p][out_slot<PR>(j)];
-            const cf32 across = lane_value(v[p][out_slot<PR>(PR::E - 1 - j)], mirror);
-            const cf32 zm = lane == 0 ? v[p][out_slot<PR>((PR::E - j) % PR::E)] : across;
+            const cf32 zk = u[out_slot<PR>(j)];
+            const cf32 across = lane_value(u[out_slot<PR>(PR::E - 1 - j)], mirror);
+            const cf32 zm = lane == 0 ? u[out_slot<PR>((PR::E - j) % PR::E)] : across;
             const int k = lane + j * PR::L;
             if (k < w) {
                 const cf32 ev{0.5f * (zk.re + zm.re), 0.5f * (zk.im - zm.im)};
@@ -124,6 +162,9 @@ __global__ void __launch_bounds__(F::NT)
                 trow[k] = cadd(ev, cmul(j == 0 ? base : cmul(base, c), od));
             }
         });
+        if constexpr (p + F::kAhead < F::kPasses) {
+            fetch(std::integral_constant<int, p + F::kAhead>{});
+        }
     });
     __syncthreads();
 
@@ -251,7 +292,6 @@ __global__ void __launch_bounds__(F::NT)
     constexpr int R0 = PR::template radix<0>();
     const int lane = tid % PR::L;
     const int prow = tid / PR::L;
-    cf32* const s = lds + prow * F::TR;
     cf32* const out = z + array * F::N1 * F::M;
     const cf32 base = twiddle_of<2 * F::M, true>(lane);
 #pragma unroll 1
@@ -278,7 +318,7 @@ __global__ void __launch_bounds__(F::NT)
             const cf32 od = cmul(d, off == 0 ? base : cmul(base, c));
             v[e] = cf32{ev.re - od.im, ev.im + od.re};
         });
-        run_stages<PR, 0, true, F::kTable, RowExchange<PR, F::TR>>(v, s, lane, table);
+        modes_row<F, true>(v, lds, prow, lane, table);
         if constexpr (PR::L >= 16) {
             // Rows of 16 lanes or more: every store is a run of at least 128 bytes.
             cf32* const dst = out + row * F::M;
@@ -295,7 +335,7 @@ __global__ void __launch_bounds__(F::NT)
             // Short rows: back to the scratch, then each wave stores its 64 / L consecutive rows
             // (consecutive in z too) as one contiguous run.
             lds_sync<true>();
-            final_write<PR>(s, v, lane);
+            final_write<PR>(lds + prow * F::TR, v, lane);
             lds_sync<true>();
             constexpr int kWaveRows = 64 / PR::L;
             const int r0 = (tid / 64) * kWaveRows;  // first scratch row of this wave

@@ -87,6 +87,8 @@ struct Fused2dFns {
                            hipStream_t stream);
     void (*c2r_transposed)(const cf32* x, float* y, cf32* work, int n1, int n2, int batch,
                            hipStream_t stream);
+    // Shapes beyond supports() whose pruned transforms r2c and c2r take.
+    bool (*modes_supports)(int n1, int n2, int m1, int w, int batch);
 };
 
 // The radio callers (rf.hpp): windowed spectrum of back-to-back frames, and overlap-save FIR.

@@ -90,7 +90,9 @@ ModesPlan plan_modes(const FftImpl& impl, int n1, int n2, int m1, int m2, int ba
 
     ModesPlan p{ModesRoute::Transposes, n1, n2, m1, m2, batch, n2 / 2 + 1, 0, 0, 0};
     p.narrow = values(n1, m2, batch);
-    if (impl.fused != nullptr && impl.fused->supports(n1, n2)) {
+    if (impl.fused != nullptr
+        && (impl.fused->supports(n1, n2)
+            || impl.fused->modes_supports(n1, n2, m1, m2, batch))) {
         p.route = ModesRoute::SinglePass;
     } else if (impl.pruned != nullptr) {
         p.route = ModesRoute::InKernel;

@@ -676,6 +676,49 @@ __device__ __forceinline__ void run_stages(cf32 (&v)[P::E], cf32* s, int lane, c
     }
 }
 
+// The same exchanges through half the LDS: a transform's scratch holds one float per element, the
+// real parts cross first and the imaginary parts after them. Where the scratch bounds the workgroups
+// of a compute unit or the rows of a pass, for twice the (half as wide) LDS instructions.
+template <class P, int S, class Lay, bool Im>
+__device__ __forceinline__ void stage_exchange_part(float* s, cf32 (&v)[P::E], int lane)
+{
+    constexpr int R = P::template radix<S>();
+    constexpr int NS = P::template span_before<S>();
+    constexpr int RN = P::template radix<S + 1>();
+    static_assert(write_splits<P, Lay>(R, NS) && read_splits<P, Lay>(RN),
+                  "LDS offsets do not split for this plan");
+    const int k0 = lane & (NS - 1);
+    float* const to = s + Lay::at((lane - k0) * R + k0);
+    const float* const from = s + Lay::at(lane);
+    lds_sync<P::kWaveLocal>();  // every lane has read the previous contents of s
+    static_for<0, P::E>([&](auto ei) {
+        constexpr int b = decltype(ei)::value / R;
+        constexpr int r = decltype(ei)::value % R;
+        constexpr int kb = (b * P::L) % NS;
+        const cf32 x = v[b * R + r];
+        to[Lay::at((b * P::L - kb) * R + kb + r * NS)] = Im ? x.im : x.re;
+    });
+    lds_sync<P::kWaveLocal>();
+    static_for<0, P::E>([&](auto ei) {
+        constexpr int b = decltype(ei)::value / RN;
+        constexpr int r = decltype(ei)::value % RN;
+        const float x = from[Lay::at(b * P::L + r * (P::N / RN))];
+        (Im ? v[b * RN + r].im : v[b * RN + r].re) = x;
+    });
+}
+
+template <class P, int S, bool Inv, bool Table, class Lay = Padded>
+__device__ __forceinline__ void run_stages_split(cf32 (&v)[P::E], float* s, int lane,
+                                                 const cf32* table)
+{
+    stage_compute<P, S, Inv, Table>(v, lane, table);
+    if constexpr (S + 1 < P::kStages) {
+        stage_exchange_part<P, S, Lay, false>(s, v, lane);
+        stage_exchange_part<P, S, Lay, true>(s, v, lane);
+        run_stages_split<P, S + 1, Inv, Table, Lay>(v, s, lane, table);
+    }
+}
+
 // Slot of the first stage's inputs that holds the element the last stage leaves in slot e_out.
 // Both hold the same elements of a lane, lane + q L for q < E (b L + r N / R covers every q
 // once at any radix), in different register orders: a transform's output can feed another

@@ -1043,6 +1043,10 @@ struct Stockham {
 #define SPX_MODES_SHAPES(X)                                                                     \
     X(64, 64) X(128, 64) X(32, 128) X(64, 128) X(128, 128) X(32, 256) X(64, 256)
 
+// Shapes with the narrow-tile kernels only: an array's kept columns fit one workgroup's LDS where
+// its half spectrum does not.
+#define SPX_MODES_ONLY_SHAPES(X) X(256, 256) X(128, 256) X(256, 128)
+
 template <int N1, int N2>
 constexpr bool modes_shape()
 {
@@ -1069,10 +1073,25 @@ struct Fused2dDriver {
         return false;
     }
 
+    // The shapes beyond those whose pruned transforms with w <= n2/8 take a narrow-tile kernel. One
+    // workgroup per array: 256 x 256 arrays take 10 to 12 us however few there are, against 10.6 us
+    // for 32 and 12.6 to 13.4 us for 64 in two passes (one array: two short launches), so they
+    // need 48; the smaller shapes (7 us against 10 us for one array) always win.
+    static bool modes_supports(int n1, int n2, int m1, int w, int batch)
+    {
+        if constexpr (R >= 4) {
+#define SPX_X(A, B) || (n1 == (A) && n2 == (B))
+            return (false SPX_MODES_ONLY_SHAPES(SPX_X)) && m1 > 0 && w <= n2 / 8
+                   && (n1 * n2 < 65536 || batch >= 48);
+#undef SPX_X
+        }
+        return false;
+    }
+
     static void check(const void* real_side, const void* complex_side, int n1, int n2, int m1,
                       int w, int batch)
     {
-        if (!supports(n1, n2)) {
+        if (!supports(n1, n2) && !modes_supports(n1, n2, m1, w, batch)) {
             throw InvalidArgument("fused 2D: no kernel for " + str(n1) + " x " + str(n2));
         }
         if (batch < 1 || m1 < 0 || 2 * m1 > n1 || w < 1 || w > n2 / 2 + 1) {
@@ -1090,17 +1109,60 @@ struct Fused2dDriver {
         }
     }
 
+    // The narrow-tile kernels (w <= W <= n2/8 kept columns, m1 > 0). Where the full width's tile
+    // leaves room for one workgroup per compute unit, half the width takes a tile for two.
+    template <int N1, int M, int W = M / 4>
+    static void launch_modes_r2c(const float* x, cf32* y, int m1, int w, int batch,
+                                 hipStream_t stream)
+    {
+        using F = dev::Modes2d<N1, M, R, Table, false, W>;
+        if constexpr (F::NT == 1024) {
+            if (w <= W / 2) {
+                launch_modes_r2c<N1, M, W / 2>(x, y, m1, w, batch, stream);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((dev::rfft2_modes_kernel<F>), dim3(static_cast<unsigned>(batch)),
+                           dim3(F::NT), 0, stream, reinterpret_cast<const cf32*>(x), y, m1, w,
+                           dev::FastDiv::of(static_cast<unsigned>(w)),
+                           Table ? twiddle_table() : nullptr);
+        SPX_LAUNCH_CHECK();
+    }
+
+    template <int N1, int M, int W = M / 4>
+    static void launch_modes_c2r(const cf32* x, float* y, int m1, int w, int batch,
+                                 hipStream_t stream)
+    {
+        using F = dev::Modes2d<N1, M, R, Table, true, W>;
+        if constexpr (F::NT == 1024) {
+            if (w <= W / 2) {
+                launch_modes_c2r<N1, M, W / 2>(x, y, m1, w, batch, stream);
+                return;
+            }
+        }
+        // Compile-time bounds on w (half the tile's columns, or all of them) and on m1 (an
+        // eighth, a quarter or half of the rows): the smallest that hold them.
+        const auto pick = [m1](auto wb) {
+            constexpr int kW = decltype(wb)::value;
+            return m1 <= N1 / 8   ? dev::irfft2_modes_kernel<F, kW, N1 / 8>
+                   : m1 <= N1 / 4 ? dev::irfft2_modes_kernel<F, kW, N1 / 4>
+                                  : dev::irfft2_modes_kernel<F, kW, N1 / 2>;
+        };
+        const auto kernel = w <= F::WMax / 2 ? pick(std::integral_constant<int, F::WMax / 2>{})
+                                             : pick(std::integral_constant<int, F::WMax>{});
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(batch)), dim3(F::NT), 0, stream, x,
+                           reinterpret_cast<cf32*>(y), m1, w,
+                           dev::FastDiv::of(static_cast<unsigned>(w)),
+                           Table ? twiddle_table() : nullptr);
+        SPX_LAUNCH_CHECK();
+    }
+
     template <int N1, int M>
     static void launch_r2c(const float* x, cf32* y, int m1, int w, int batch, hipStream_t stream)
     {
         if constexpr (modes_shape<N1, 2 * M>()) {
             if (m1 > 0 && w <= M / 4) {
-                using F = dev::Modes2d<N1, M, R, Table>;
-                hipLaunchKernelGGL((dev::rfft2_modes_kernel<F>), dim3(static_cast<unsigned>(batch)),
-                                   dim3(F::NT), 0, stream, reinterpret_cast<const cf32*>(x), y, m1,
-                                   w, dev::FastDiv::of(static_cast<unsigned>(w)),
-                                   Table ? twiddle_table() : nullptr);
-                SPX_LAUNCH_CHECK();
+                launch_modes_r2c<N1, M>(x, y, m1, w, batch, stream);
                 return;
             }
         }
@@ -1125,23 +1187,7 @@ struct Fused2dDriver {
     {
         if constexpr (modes_shape<N1, 2 * M>()) {
             if (m1 > 0 && w <= M / 4) {
-                using F = dev::Modes2d<N1, M, R, Table>;
-                // Compile-time bounds on w (half the tile's columns, or all of them) and on m1
-                // (an eighth, a quarter or half of the rows): the smallest that hold them.
-                const auto pick = [m1](auto wb) {
-                    constexpr int kW = decltype(wb)::value;
-                    return m1 <= N1 / 8   ? dev::irfft2_modes_kernel<F, kW, N1 / 8>
-                           : m1 <= N1 / 4 ? dev::irfft2_modes_kernel<F, kW, N1 / 4>
-                                          : dev::irfft2_modes_kernel<F, kW, N1 / 2>;
-                };
-                const auto kernel = w <= F::WMax / 2
-                                        ? pick(std::integral_constant<int, F::WMax / 2>{})
-                                        : pick(std::integral_constant<int, F::WMax>{});
-                hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(batch)), dim3(F::NT), 0,
-                                   stream, x, reinterpret_cast<cf32*>(y), m1, w,
-                                   dev::FastDiv::of(static_cast<unsigned>(w)),
-                                   Table ? twiddle_table() : nullptr);
-                SPX_LAUNCH_CHECK();
+                launch_modes_c2r<N1, M>(x, y, m1, w, batch, stream);
                 return;
             }
         }
@@ -1178,6 +1224,13 @@ struct Fused2dDriver {
         return;                                                      \
     }
             SPX_FUSED_SHAPES(SPX_X)
+#undef SPX_X
+#define SPX_X(A, B)                                                  \
+    if (n1 == (A) && n2 == (B)) {                                    \
+        launch_modes_r2c<(A), (B) / 2>(x, y, m1, w, batch, stream);  \
+        return;                                                      \
+    }
+            SPX_MODES_ONLY_SHAPES(SPX_X)
 #undef SPX_X
         }
     }
@@ -1372,9 +1425,10 @@ struct Fused2dDriver {
 
     static Fused2dFns fns()
     {
-        return {&supports,       &r2c,           &c2r,           &r2c_columns, &r2c_rows,
-                &c2r_rows,       &c2c_supports,  &c2c,           &c2c_rows,    &c2c_transposed,
-                &r2c_transposed, &c2r_transposed};
+        return {&supports,       &r2c,            &c2r,           &r2c_columns,
+                &r2c_rows,       &c2r_rows,       &c2c_supports,  &c2c,
+                &c2c_rows,       &c2c_transposed, &r2c_transposed, &c2r_transposed,
+                &modes_supports};
     }
 
     static void c2r(const cf32* x, float* y, int n1, int n2, int m1, int w, int batch,
@@ -1388,6 +1442,13 @@ struct Fused2dDriver {
         return;                                                      \
     }
             SPX_FUSED_SHAPES(SPX_X)
+#undef SPX_X
+#define SPX_X(A, B)                                                  \
+    if (n1 == (A) && n2 == (B)) {                                    \
+        launch_modes_c2r<(A), (B) / 2>(x, y, m1, w, batch, stream);  \
+        return;                                                      \
+    }
+            SPX_MODES_ONLY_SHAPES(SPX_X)
 #undef SPX_X
         }
     }

@@ -117,6 +117,30 @@ def test_narrow_tile_kernels_at_their_bounds(rng, impl, n1, n2, m1, m2):
     assert_transform_close(back, ref.irfft2_from_modes(modes, (n1, n2)), n1 * n2, axes=AXES)
 
 
+# The same bounds for the shapes whose half spectrum does not fit one workgroup but whose kept
+# columns do, and the first width past them, back on two passes.
+@pytest.mark.parametrize("impl", ["stockham_r4", "stockham_r8", "stockham_r8_table"])
+@pytest.mark.parametrize(("n1", "n2"), [(256, 256), (128, 256), (256, 128)])
+@pytest.mark.parametrize(("m1_of", "m2_of"), [(lambda n: 1, lambda n: 1),
+                                              (lambda n: n // 8, lambda n: n // 16),
+                                              (lambda n: n // 8 + 1, lambda n: n // 16 + 1),
+                                              (lambda n: n // 4 + 1, lambda n: n // 8 - 1),
+                                              (lambda n: n // 2, lambda n: n // 8),
+                                              (lambda n: n // 4, lambda n: n // 8 + 1)])
+def test_large_narrow_tile_kernels(rng, impl, n1, n2, m1_of, m2_of):
+    m1, m2 = m1_of(n1), m2_of(n2)
+    batch = 49 if n1 * n2 == 65536 else 3  # fewer than 48 arrays of 256 x 256 take two passes
+    x = random_real(rng, (batch, n1, n2))
+    y = spectral.rfft2_truncated(dev(x), m1, m2, impl=impl)
+    assert_transform_close(y, ref.rfft2_truncate(x, m1, m2), n1 * n2, axes=AXES)
+    modes = random_complex(rng, (batch, 2 * m1, m2))
+    back = spectral.irfft2_from_modes(dev(modes), (n1, n2), impl=impl)
+    assert_transform_close(back, ref.irfft2_from_modes(modes, (n1, n2)), n1 * n2, axes=AXES)
+    for few in (1, 47):  # the other side of the rule
+        assert_transform_close(spectral.rfft2_truncated(dev(x[:few]), m1, m2, impl=impl),
+                               ref.rfft2_truncate(x[:few], m1, m2), n1 * n2, axes=AXES)
+
+
 # --- the mode layout, bit for bit ------------------------------------------------------------
 
 @pytest.mark.parametrize("impl", IMPLS)
