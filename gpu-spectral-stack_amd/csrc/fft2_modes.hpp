@@ -10,9 +10,10 @@
 // column tile (N1 rows by TC >= w values): at 128 x 128 with w <= 16, 40 KB, so four arrays share
 // a CU and more of the HBM traffic overlaps the transforms.
 //
-//   forward  the row passes' loads first, as many passes as fit 32 values per lane, then per pass: row transform (exchanges in the
-//            scratch), bins X[k], k < w, into the tile; the w columns in place down the tile;
-//            the kept rows (0 .. m1-1, n1-m1 .. n1-1) of those columns stored flat.
+//   forward  the row passes' loads first, as many passes as fit 32 values per lane, then per
+//            pass: row transform (exchanges in the scratch), bins X[k], k < w, into the tile; the
+//            w columns in place down the tile; the kept rows (0 .. m1-1, n1-m1 .. n1-1) of those
+//            columns stored flat.
 //   inverse  the kept modes into the tile (the other rows read as zeros); inverse columns; per
 //            pass: each lane forms its row-inverse inputs straight from the tile row (the c2r
 //            prepare), inverse row transform, the real rows stored.

@@ -11,6 +11,7 @@
 #include "fft2_modes.hpp"
 #include "fft2_pairs.hpp"
 #include "fft2_transposed.hpp"
+#include "fft_split.hpp"
 #include "fft_api.hpp"
 #include "rf.hpp"
 #include "stockham.hpp"
@@ -185,6 +186,32 @@ inline constexpr bool kFusedPersistent = SPX_FUSED_PERSISTENT != 0;
 #endif
 inline constexpr bool kPersistentLarge = SPX_LARGE_PERSISTENT != 0;
 
+// Unpruned columns of 1024 and 2048 points, radix-8 variants: tiles of 16 columns in registers
+// (fft_split.hpp). At 1024 points from 64 tiles on: the persistent kernel's 8-column tiles are twice
+// as many and less work each, and keep the small batches (2 tiles 15.3 against 13.7 us for an
+// rfft2; 64 tiles 14.5 against 14.2 us; 256 tiles 16.2 against 21.4 us; 1024 tiles, 2^24 points,
+// 58.7 against 69.9 us). At 2048 points wherever the columns ran as two passes: 2048 x 64 arrays,
+// fft2, one 29.3 -> 20.2 us, 64 of them 72.5 -> 53.5 us.
+template <int N, int R>
+bool split_columns(const StridedIo& io, long long batch)
+{
+    if constexpr (R == 8 && kRadix16) {
+        return io.m1_in == 0 && io.m1_out == 0 && io.cols >= (N == 1024 ? 16 : 32)
+               && batch >= (N == 1024 ? 64 : 1) * SplitColumnPlan<N>::kTile;
+    }
+    return false;
+}
+
+template <int N, bool Inv, bool Table>
+void launch_split_columns(const StridedIo& io, long long batch, hipStream_t stream)
+{
+    using P = SplitColumnPlan<N>;
+    const long long tiles = (batch + P::kTile - 1) / P::kTile;
+    hipLaunchKernelGGL((columns_split_kernel<P, Inv, Table>), dim3(static_cast<unsigned>(tiles)),
+                       dim3(P::kLanes), 0, stream, io, batch, Table ? twiddle_table() : nullptr);
+    SPX_LAUNCH_CHECK();
+}
+
 // Strided columns of 256, 512 and 1024 points, and of 64 and 128 points in wide matrices, run
 // persistent (columns_kernel); other lengths keep one tile per workgroup. The 1024-point tiles hold
 // 8 columns of 16 values per lane, one wave per column (workgroups of 512 lanes), in XCD order:
@@ -228,7 +255,22 @@ void dispatch_strided_columns(int n, const StridedIo& io, long long batch, hipSt
         launch_columns_persistent<Plan<512, R, column_e<512, R>(), column_threads<512, R>()>, Inv,
                                   Table>(io, batch, stream);
         break;
+    case 2048:
+        if constexpr (R == 8 && kRadix16) {
+            if (split_columns<2048, R>(io, batch)) {
+                launch_split_columns<2048, Inv, Table>(io, batch, stream);
+                break;
+            }
+        }
+        dispatch_columns<R, Inv, Table>(n, io, batch, stream);
+        break;
     case 1024:
+        if constexpr (R == 8 && kRadix16) {
+            if (split_columns<1024, R>(io, batch)) {
+                launch_split_columns<1024, Inv, Table>(io, batch, stream);
+                break;
+            }
+        }
         // Radix 16 in the radix-8 variants (two exchanges instead of three): the 2^20-point
         // C2C over 2^24 points 115.6 -> 112.0 us in interleaved runs.
         launch_columns_persistent<Plan<1024, (R == 8 ? 16 : R), 16, 512>, Inv, Table, 32>(
@@ -677,13 +719,19 @@ struct Stockham {
         }
     }
 
-    // n = n1 x n2 in two passes, for kSinglePassMaxN < n <= kTwoPassMaxN: n1-point transforms down
+    // Columns of 2048 points and twiddled rows of 2048 points run in one pass (fft_split.hpp), so
+    // two passes reach 2^22 points.
+    static constexpr bool kSplit = R == 8 && dev::kRadix16;
+
+    // n = n1 x n2 in two passes, for kSinglePassMaxN < n <= kTwoPassMaxN (4 kTwoPassMaxN with
+    // kSplit: 2^21 = 2048 x 1024 134.7 -> 107 us over 2^24 points against the three passes, 2^22 =
+    // 2048 x 2048 143.0 -> 124.5 us, and no slower for one transform): n1-point transforms down
     // the n2 columns of each n1 x n2 matrix (x -> work), then the twiddled n2-point rows, stored
     // transposed (work -> y): X[k1 + n1 k2] is row k1's element k2.
     static void two_pass(const cf32* x, cf32* y, int n, int batch, Direction direction,
                          hipStream_t stream, cf32* given)
     {
-        const int n2 = n <= (1 << 18) ? 512 : 1024;
+        const int n2 = n <= (1 << 18) ? 512 : n <= (1 << 21) ? 1024 : 2048;
         const int n1 = n / n2;
         if (static_cast<long long>(batch) * n1 > INT_MAX
             || static_cast<long long>(batch) * n2 > INT_MAX) {
@@ -700,8 +748,10 @@ struct Stockham {
         const long long transforms = static_cast<long long>(batch) * n1;
         if (n2 == 512) {
             launch_rows<512>(rows, inverse, transforms, stream);
-        } else {
+        } else if (n2 == 1024) {
             launch_rows<1024>(rows, inverse, transforms, stream);
+        } else if constexpr (kSplit) {
+            launch_rows<2048>(rows, inverse, transforms, stream);
         }
     }
 
@@ -709,16 +759,27 @@ struct Stockham {
     static void launch_rows(const dev::TwiddleRowsTransposedIo& rows, bool inverse,
                             long long transforms, hipStream_t stream)
     {
-        using P = dev::TransposedRowsPlan<N2, R>;
-        if (inverse) {
-            dev::launch<P, true, Table>(rows, transforms, stream);
+        if constexpr (N2 == 2048) {
+            using P = dev::SplitPlan<N2>;
+            using Io = dev::TwiddleRowsTransposedIo;
+            const auto kernel = inverse ? dev::rows_split_kernel<P, true, Table, Io>
+                                        : dev::rows_split_kernel<P, false, Table, Io>;
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(transforms / P::kTile)),
+                               dim3(P::kLanes), 0, stream, rows,
+                               Table ? twiddle_table() : nullptr);
+            SPX_LAUNCH_CHECK();
         } else {
-            dev::launch<P, false, Table>(rows, transforms, stream);
+            using P = dev::TransposedRowsPlan<N2, R>;
+            if (inverse) {
+                dev::launch<P, true, Table>(rows, transforms, stream);
+            } else {
+                dev::launch<P, false, Table>(rows, transforms, stream);
+            }
         }
     }
 
-    // Any power of two up to kFourStepMaxN: one kernel up to kSinglePassMaxN, two passes up to
-    // kTwoPassMaxN, three beyond.
+    // Any power of two up to kFourStepMaxN: one kernel up to kSinglePassMaxN, then two passes
+    // (two_pass), then three.
     // work: nullptr, or the caller's scratch of c2c_scratch_values(n, batch) values.
     static void c2c(const cf32* x, cf32* y, int n, int batch, Direction direction,
                     hipStream_t stream, cf32* work = nullptr)
@@ -748,7 +809,7 @@ struct Stockham {
             }
             return;
         }
-        if (n <= kTwoPassMaxN) {
+        if (n <= (kSplit ? 4 * kTwoPassMaxN : kTwoPassMaxN)) {
             two_pass(x, y, n, batch, direction, stream, work);
             return;
         }
@@ -814,7 +875,7 @@ struct Stockham {
         launch_rows<n2>(rows, inverse, static_cast<long long>(batch) * n1, stream);
     }
 
-    // Columns of n = 2048 or 4096 points as two passes of 64 x (n / 64) (a four-step split of
+    // Columns of n = 2048 (without kSplit) or 4096 points as two passes of 64 x (n / 64) (a four-step split of
     // the column axis): a single pass would stage only 4 or 2 columns per workgroup, reading
     // runs of 32 or 16 bytes; each of these passes stages 32 columns of 64 points (256-byte
     // runs). Pass A runs
@@ -887,7 +948,7 @@ struct Stockham {
             throw InvalidArgument("stockham columns: a pruned transform cannot run in place");
         }
         const long long batch = static_cast<long long>(cols) * slabs;
-        if (n >= 2048 && m1_in == 0 && m1_out == 0 && cols >= 32) {
+        if (n >= 2048 && m1_in == 0 && m1_out == 0 && cols >= 32 && !(kSplit && n == 2048)) {
             long_columns(x, y, n, cols, slabs, direction, stream, stream_out);
             return;
         }

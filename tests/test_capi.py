@@ -450,6 +450,29 @@ def test_direct_columns_over_many_tiles(lib, rng, n, slabs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("inverse", [0, 1])
+@pytest.mark.parametrize(("n", "cols", "slabs"), [(1024, 16, 63), (1024, 16, 64), (1024, 17, 61),
+                                                  (1024, 33, 33), (1024, 15, 80), (2048, 31, 3),
+                                                  (2048, 32, 1), (2048, 33, 3), (2048, 100, 2)])
+def test_long_columns_in_register_tiles(lib, rng, n, cols, slabs, inverse):
+    # Columns of 1024 points (from 64 tiles of 16 columns on) and of 2048 points, 16 to a tile in
+    # registers: whole and partial last tiles, tiles over two slabs, and both sides of the rule.
+    from oracle.tolerance import assert_transform_close, random_complex
+
+    x = random_complex(rng, (slabs, n, cols))
+    xd = torch.from_numpy(x).cuda()
+    guard = torch.full((slabs * n * cols + 64,), 7.0, dtype=torch.complex64, device="cuda")
+    yd = guard[: xd.numel()].view_as(xd)
+    assert lib.spx_columns(3, _ptr(xd), _ptr(yd), n, cols, slabs, inverse, None) == SPX_OK
+    inplace = xd.clone()
+    assert lib.spx_columns(3, _ptr(inplace), _ptr(inplace), n, cols, slabs, inverse, None) == SPX_OK
+    torch.cuda.synchronize()
+    assert_transform_close(yd, _fft_columns(x, bool(inverse)), n, axes=(-2,))
+    assert torch.equal(inplace, yd)
+    assert bool((guard[xd.numel():] == 7.0).all())  # nothing past the last column
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [256, 512, 1024, 2048, 4096, 8192])
 def test_direct_pruned_r2c_at_every_row_width(lib, rng, n):
     # R2C rows of 16 .. 256 lanes at radix 8: the register combine with the staged store (16, 32
