@@ -66,6 +66,7 @@ CAPI_SOURCES = [
     "noalloc.hip",
     "fft2d.hip",
     "pruned.hip",
+    "fir_direct.hip",
     "ns.hip",
     "ns_grid.hip",
     "registry.cpp",

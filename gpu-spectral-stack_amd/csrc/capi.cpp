@@ -395,6 +395,14 @@ int spx_rf_fir(int impl, const void* x, const void* h, void* y, long long n, int
     });
 }
 
+int spx_rf_fir_direct_taps(void) { return spx::kFirDirectTaps; }
+
+int spx_rf_fir_direct(const void* x, const float* taps, void* y, long long n, int count,
+                      long long rows, hipStream_t stream)
+{
+    return guarded([&] { spx::fir_direct(cc(x), taps, cm(y), n, count, rows, stream); });
+}
+
 int spx_rf_fir_spectrum(int impl, const void* taps, int complex_taps, void* h, int count,
                         int nfft, hipStream_t stream)
 {

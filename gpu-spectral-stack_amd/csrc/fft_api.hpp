@@ -106,6 +106,12 @@ struct RfFns {
     int max_nfft;
 };
 
+// Short real filters (fir_direct.hip), for any implementation: y (rows, n) = x filtered by `count`
+// float taps, 1 <= count <= kFirDirectTaps.
+constexpr int kFirDirectTaps = 129;
+void fir_direct(const cf32* x, const float* taps, cf32* y, long long n, int count,
+                long long rows, hipStream_t stream);
+
 // One implementation, by name (reference registry.hpp:14-25).
 struct FftImpl {
     const char* name;

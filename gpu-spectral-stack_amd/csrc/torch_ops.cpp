@@ -17,6 +17,7 @@
 
 #include "spectral_hip.h"
 
+#include <algorithm>
 #include <climits>
 #include <cstdint>
 #include <optional>
@@ -469,6 +470,28 @@ at::Tensor rf_fir_spectrum_op(const at::Tensor& taps, int64_t nfft, c10::string_
     return h;
 }
 
+// The FIR from its float32 taps (at most spx_rf_fir_direct_taps()), one launch.
+at::Tensor rf_fir_direct_op(const at::Tensor& x, const at::Tensor& taps)
+{
+    check_complex64_cuda(x, "x");
+    TORCH_CHECK(x.dim() >= 1, "rf_fir_direct: x needs at least one dimension");
+    TORCH_CHECK_VALUE(taps.is_cuda() && taps.scalar_type() == at::kFloat && taps.dim() == 1
+                          && taps.device() == x.device(),
+                      "taps must be a 1D float32 CUDA tensor on x's device");
+    at::Tensor y = at::empty(x.sizes(), x.options());
+    const int64_t n = x.size(-1);
+    if (x.numel() == 0) {
+        return y;
+    }
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const at::Tensor xc = x.contiguous();
+    const at::Tensor tc = taps.contiguous();
+    const auto count = static_cast<int>(std::min<int64_t>(tc.numel(), INT_MAX));
+    check_status(spx_rf_fir_direct(cptr(xc), tc.const_data_ptr<float>(), mptr(y), n, count,
+                                   x.numel() / n, current_stream()));
+    return y;
+}
+
 // --- the Navier-Stokes caller: one fused IMEX stage per field (no reference operator; the
 // reference's GpuSolver composes its transforms with torch elementwise ops instead) ----------
 
@@ -645,12 +668,20 @@ PyObject* py_ns_grid_supports(PyObject*, PyObject* arg)
                            && spx_ns_grid_supports(static_cast<int>(n)) == 1);
 }
 
+// spectral._C.rf_fir_direct_taps(): the longest filter rf_fir_direct takes.
+PyObject* py_rf_fir_direct_taps(PyObject*, PyObject*)
+{
+    return PyLong_FromLong(spx_rf_fir_direct_taps());
+}
+
 PyMethodDef module_methods[] = {
     {"fft_impls", py_fft_impls, METH_NOARGS, "Names of the FFT implementations, in order."},
     {"ns_supports", py_ns_supports, METH_O,
      "Whether the fused Navier-Stokes stage has a kernel for an n x n grid."},
     {"ns_grid_supports", py_ns_grid_supports, METH_O,
      "Whether ns_advance_grid takes an n x n grid."},
+    {"rf_fir_direct_taps", py_rf_fir_direct_taps, METH_NOARGS,
+     "The longest filter rf_fir_direct takes."},
     {nullptr, nullptr, 0, nullptr},
 };
 
@@ -674,6 +705,7 @@ TORCH_LIBRARY(spectral, m)
     m.def("rf_spectrum(Tensor x, Tensor? window, int nfft, str impl) -> Tensor");
     m.def("rf_fir(Tensor x, Tensor h, int taps, int nfft, str impl) -> Tensor");
     m.def("rf_fir_spectrum(Tensor taps, int nfft, str impl) -> Tensor");
+    m.def("rf_fir_direct(Tensor x, Tensor taps) -> Tensor");
     // The Navier-Stokes caller's fused stages (no reference operator).
     m.def("ns_predict(Tensor w_hat, Tensor forcing_hat, Tensor nu, float drag, float dt, int n)"
           " -> (Tensor, Tensor)");
@@ -700,6 +732,7 @@ TORCH_LIBRARY_IMPL(spectral, CUDA, m)
     m.impl("rf_spectrum", &rf_spectrum_op);
     m.impl("rf_fir", &rf_fir_op);
     m.impl("rf_fir_spectrum", &rf_fir_spectrum_op);
+    m.impl("rf_fir_direct", &rf_fir_direct_op);
     m.impl("ns_predict", &ns_predict_op);
     m.impl("ns_correct", &ns_correct_op);
     m.impl("ns_advance", &ns_advance_op);

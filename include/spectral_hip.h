@@ -199,7 +199,12 @@ int spx_ns_grid_steps(const void* w_in, void* w_out, void* work, const void* for
  *                    forward FFT of the taps zero-padded to nfft (complex64).
  *   spx_rf_fir_spectrum  that h from `count` taps (float32, or complex64 when complex_taps != 0),
  *                    1 <= count <= nfft, in one launch; it replaces rf.py:145-147 (zeros, a copy
- *                    of the converted taps, fft). */
+ *                    of the converted taps, fft).
+ *   spx_rf_fir_direct  the same y from the taps themselves, 1 <= count <= spx_rf_fir_direct_taps()
+ *                    float32 values: the convolution sum on the matrix cores, no blocks. */
+int spx_rf_fir_direct_taps(void);
+int spx_rf_fir_direct(const void* x, const float* taps, void* y, long long n, int count,
+                      long long rows, hipStream_t stream);
 int spx_rf_max_nfft(int impl);
 int spx_rf_spectrum(int impl, const void* x, const float* window, void* y, long long n, int nfft,
                     long long rows, hipStream_t stream);

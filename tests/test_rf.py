@@ -384,3 +384,40 @@ def test_command_line_spectrum_writes_every_frame(tmp_path):
     written = rf.read_cf32(out).reshape(-1, 512)
     assert written.shape[0] == -(-len(samples) // 512)
     assert rel_l2(written, framed_spectrum(samples, 512, "hann")) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("taps", [1, 2, 16, 17, 18, 63, 64, 65, 112, 113, 114, 129, 130])
+@pytest.mark.parametrize("shape", [(1,), (15,), (1023,), (1024,), (1025,), (3, 2048), (5, 2500),
+                                   (2, 1024 * 1024 + 70)])
+def test_short_real_filters_match_the_convolution_sum(rng, taps, shape):
+    # The sum on the matrix cores (up to 129 taps, 64 beyond 2^20 samples) and the blocks past those
+    # lengths: steps of 1024 outputs whole and partial, first steps, rows, windows of 16 j samples.
+    x = (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).astype(np.complex64)
+    h = rng.standard_normal(taps).astype(np.float32)
+    y = rf.fir(torch.from_numpy(x).cuda(), torch.from_numpy(h), fft_impl="stockham_r8")
+    expected = scipy.signal.lfilter(h.astype(np.float64), 1.0, x.astype(np.complex128), axis=-1)
+    got = y.cpu().numpy()
+    # Each output sums `taps` products: their rounding is below taps eps32 times the sum's scale.
+    scale = np.abs(h).sum() * np.abs(x).max()
+    assert got.shape == shape and np.abs(got - expected).max() <= taps * 1.2e-7 * scale + 1e-6 * scale
+
+
+@pytest.mark.gpu
+def test_short_real_filters_keep_the_calls_rules(rng):
+    x = torch.from_numpy((rng.standard_normal((4, 3000)) * (1 + 1j)).astype(np.complex64)).cuda()
+    h = torch.from_numpy(rng.standard_normal(31))  # float64 on the host
+    y = rf.fir(x, h, fft_impl="stockham_r8")
+    blocks = rf.fir(x, h, nfft=256, fft_impl="stockham_r8")
+    assert torch.linalg.norm(y - blocks) < 1e-6 * torch.linalg.norm(blocks)
+    assert torch.equal(rf.fir(x.T.contiguous().T, h, fft_impl="stockham_r8"), y)  # any strides
+    assert rf.fir(x[:0], h, fft_impl="stockham_r8").shape == (0, 3000)
+    # An infinity reaches only the outputs of its own 16-sample windows.
+    x[1, 2000] = float("inf")
+    z = rf.fir(x, h, fft_impl="stockham_r8")
+    assert torch.isfinite(torch.view_as_real(z[1, :1984])).all()
+    assert torch.isfinite(torch.view_as_real(z[1, 2064:])).all() and torch.equal(z[0], y[0])
+    with pytest.raises(ValueError, match="1 to 129"):
+        torch.ops.spectral.rf_fir_direct(x, torch.ones(130, device="cuda"))
+    with pytest.raises(ValueError, match="float32"):
+        torch.ops.spectral.rf_fir_direct(x, h.cuda())
