@@ -12,25 +12,28 @@
 // row spectrum is P[k] = (A~ + i B~)[k] at k >= 0 and Q[k] = conj((A~ - i B~)[k]) at -k, and as
 // the column transforms are linear, P and Q are column transforms of the state times one complex
 // multiplier per mode each. Per stage:
-//   ns_columns_kernel  the inverse column transforms of P1, Q1, P2, Q2, one tile of columns of one
-//                      of them per workgroup: state -> work (field, grid row, 4, pitch)
 //   ns_rows_kernel     two grid rows per lane group: each row's z1 and z2 (n-point complex inverses
 //                      read straight from P and Q), their product, then ONE complex forward of both
-//                      rows' products, split into the two rows' first W bins: work -> work, over
-//                      the rows it read
-//   ns_update_kernel   the forward columns of those bins and the IMEX update of the kept rows
-//                        stage 0: out_f = F, out_w = (e w + dt F) i
+//                      rows' products, split into the two rows' first W bins: work -> bins
+//   ns_update_columns_kernel  the forward columns of those bins and the IMEX update of the kept
+//                      rows, then, from the same registers, the inverse column transforms of the
+//                      next stage's P1, Q1, P2, Q2: bins -> state, work (field, grid row, 4, pitch)
+//                        stage 0: out_f = F, state (e w + dt F) i, which only the columns see
 //                        stage 1: out_w = (e w0 + dt/2 (f0 + F)) i
 //                      with F = f_hat - mask N_hat, e = 1 + dt/2 L, i = 1 / (1 - dt/2 L),
 //                      L = -nu |k|^2 - alpha.
-// Every pass moves its arrays once; the derived spectra (4 n pitch values per field) are the one
-// large intermediate. Normalization: inverse 1 / n^2, forward none, as numpy. The imaginary parts
-// of a row's zero and n/2 frequencies are dropped, as numpy's irfft drops them.
+// A call's first stage takes its columns from ns_columns_kernel and its last one ends in
+// ns_update_kernel. The derived spectra (4 n pitch values per field) are the one large
+// intermediate. Normalization: inverse 1 / n^2, forward none, as numpy. The imaginary parts of a
+// row's zero and n/2 frequencies are dropped, as numpy's irfft drops them.
 //
-// Measured on MI355X (256^2 pruned, 48 fields): columns 12.8 us (38 MB written), rows 13.0 us
-// (38 MB read, 8 MB written), update 10.3 us; a stage was about 105 us composed. About 4 us of
-// each launch is its ramp and drain; neither fewer stages (radix 16) nor the update's loads issued
-// ahead of its transform moved the rest.
+// Measured on MI355X (256^2 pruned, 48 fields, six steps and a frame): 434 us with the update and
+// the columns apart (10.3 and 12.8 us; rows 13.0 us), 349 us as here (rows 13.0, update and
+// columns 17 us a launch). The update and columns are
+// bound by their instructions (about 1700 per wave, 44 waves per field), the rows by theirs and the
+// LDS exchanges; about 4 us of each launch is its ramp and drain. Rows with the second row's loads
+// ahead of the first row's transforms were 1.7 us slower (registers), with one row per lane group
+// 4 us slower (the pair's forward then runs on both).
 
 #include "stockham.hpp"
 
@@ -45,7 +48,7 @@ namespace {
 
 // A plan whose transforms span waves: the column passes hold kT neighbouring columns per tile,
 // the columns fastest over the lanes, so that every global access of a wave is whole runs of kT
-// values (128 bytes).
+// values.
 template <int N, int R, int E>
 struct ColumnPlan : Plan<N, R, E> {
     static constexpr bool kWaveLocal = false;
@@ -59,7 +62,10 @@ struct NsGrid {
     static constexpr int kRows = Pruned_ ? 2 * m : N;      // state rows per field
     static constexpr int kW = Pruned_ ? m : N / 2 + 1;     // state columns
     static constexpr int kPitch = (kW + 15) / 16 * 16;     // of P and Q rows: whole 128-byte lines
-    static constexpr int kT = N <= 512 ? 16 : 8;           // columns per tile
+    // Columns per tile. From 256 on 8, half a line per access, twice as many workgroups to balance:
+    // with both halves read on one XCD, 48 fields of 256^2 362 -> 334 us for six steps, 30 of 512^2
+    // 825 -> 722 us.
+    static constexpr int kT = N <= 128 ? 16 : 8;
     static constexpr int kTiles = (kW + kT - 1) / kT;
     // Radix and values per lane of the columns: 8 while a tile then takes at most 512 lanes. At 256
     // the update waits on its loads, not on its stages: 12.4 us with 16 values, 10.3 us with 8.
@@ -69,10 +75,12 @@ struct NsGrid {
     static constexpr int kColumnLds = pad(N - 1) * kT + kT;
     static constexpr int kRE = N <= 512 ? 8 : 16;          // rows: one wave or less per transform
     using PR = Plan<N, kRE, kRE>;
+    static constexpr int kRowParts = cmax(1, N / 2 / PR::T);  // row workgroups per field
     static constexpr int kRowLds = PR::T * PR::kStride;
 
     static_assert(PR::L <= 64 && kColumnThreads <= 1024, "workgroup shapes");
-    static_assert(slots_match<PR>(), "inverse outputs must be forward inputs");
+    static_assert(slots_match<PR>() && slots_match<PC>(),
+                  "one direction's outputs must be the other's inputs");
     static_assert(kColumnLds * sizeof(cf32) <= 80 * 1024, "two column tiles per compute unit");
 };
 
@@ -117,44 +125,50 @@ __device__ __forceinline__ cf32 multiplier(int set, float kx, float ky)
     return {(set == 2 ? -ky : ky) * kScale, kx * kScale};
 }
 
-// One tile of kT columns of one set. Blocks run set fastest within an XCD's share (consecutive
-// blocks go to consecutive XCDs), so the four sets of a tile read the state from one L2.
+// A workgroup's field and its part (0 .. Parts-1) of that field.
+struct NsBlock {
+    int field;
+    int part;
+};
+
+// Consecutive blocks go to consecutive XCDs. by_xcd: a field's blocks on one XCD; otherwise Share
+// consecutive parts on one XCD.
+template <int Parts, int Share>
+__device__ __forceinline__ NsBlock block_of(bool by_xcd)
+{
+    const int xcd = static_cast<int>(blockIdx.x) % 8;
+    const int slot = static_cast<int>(blockIdx.x) / 8;
+    if (by_xcd) {
+        return {slot / Parts * 8 + xcd, slot % Parts};
+    }
+    const int item = slot / Share * 8 + xcd;
+    return {item / (Parts / Share), item % (Parts / Share) * Share + slot % Share};
+}
+
+template <int Parts, int Share>
+unsigned blocks_of(int fields, bool by_xcd)
+{
+    return by_xcd ? static_cast<unsigned>((fields + 7) / 8) * (8u * Parts)
+                  : static_cast<unsigned>((fields * (Parts / Share) + 7) / 8) * (8u * Share);
+}
+
+// One set's inverse columns of a tile. v: the state in the transform's input slots.
 template <class G>
-__global__ void __launch_bounds__(G::kColumnThreads)
-    ns_columns_kernel(const cf32* __restrict__ state, cf32* __restrict__ work, int items)
+__device__ __forceinline__ void derived_columns(cf32 (&v)[G::PC::E], cf32* s,
+                                                cf32* __restrict__ work, int field, int col,
+                                                int lane, int set)
 {
     using P = typename G::PC;
     using Lay = PaddedRows<G::kT>;
     constexpr int R0 = P::template radix<0>();
     constexpr int RL = P::template radix<P::kStages - 1>();
-    __shared__ cf32 s[G::kColumnLds];
-    const int slot = static_cast<int>(blockIdx.x) / 8;
-    const int item = (slot / 4) * 8 + static_cast<int>(blockIdx.x) % 8;  // (field, tile)
-    const int set = slot % 4;
-    if (item >= items) {
-        return;  // the whole workgroup
-    }
-    const int field = item / G::kTiles;
-    const int tid = threadIdx.x;
-    const int c = tid % G::kT;
-    const int lane = tid / G::kT;
-    const int col = (item % G::kTiles) * G::kT + c;
-    const bool live = col < G::kW;
-    const cf32* const w = state + static_cast<long long>(field) * G::kRows * G::kW;
     const float kx = static_cast<float>(col);
-    cf32 v[P::E];
-#pragma unroll
-    for (int e = 0; e < P::E; ++e) {
-        const int i = input_index<P, 0>(lane, e / R0, e % R0);
-        const int r = state_row<G>(i);
-        v[e] = live && r >= 0 ? w[r * G::kW + col] : czero();
-    }
 #pragma unroll
     for (int e = 0; e < P::E; ++e) {
         const int i = input_index<P, 0>(lane, e / R0, e % R0);
         v[e] = cmul(v[e], multiplier<G>(set, kx, ky_of<G>(i)));
     }
-    run_stages<P, 0, true, false, Lay>(v, s + c, lane, nullptr);
+    run_stages<P, 0, true, false, Lay>(v, s, lane, nullptr);
     cf32* const out = work + (static_cast<long long>(field) * G::N * 4 + set) * G::kPitch + col;
     const float sign = (set & 1) != 0 ? -1.0f : 1.0f;
     if (col < G::kPitch) {
@@ -164,6 +178,36 @@ __global__ void __launch_bounds__(G::kColumnThreads)
             out[y * (4 * G::kPitch)] = cf32{v[e].re, sign * v[e].im};
         });
     }
+}
+
+// The first stage of a call: one tile of kT columns of one set. Blocks run set fastest within an
+// XCD's share (consecutive blocks go to consecutive XCDs), so the four sets of a tile read the state
+// from one L2.
+template <class G>
+__global__ void __launch_bounds__(G::kColumnThreads)
+    ns_columns_kernel(const cf32* __restrict__ state, cf32* __restrict__ work, int fields,
+                      bool by_xcd)
+{
+    using P = typename G::PC;
+    constexpr int R0 = P::template radix<0>();
+    __shared__ cf32 s[G::kColumnLds];
+    const auto [field, part] = block_of<4 * G::kTiles, 4>(by_xcd);
+    if (field >= fields) {
+        return;  // the whole workgroup
+    }
+    const int c = static_cast<int>(threadIdx.x) % G::kT;
+    const int lane = static_cast<int>(threadIdx.x) / G::kT;
+    const int col = part / 4 * G::kT + c;
+    const bool live = col < G::kW;
+    const cf32* const w = state + static_cast<long long>(field) * G::kRows * G::kW;
+    cf32 v[P::E];
+#pragma unroll
+    for (int e = 0; e < P::E; ++e) {
+        const int i = input_index<P, 0>(lane, e / R0, e % R0);
+        const int r = state_row<G>(i);
+        v[e] = live && r >= 0 ? w[r * G::kW + col] : czero();
+    }
+    derived_columns<G>(v, s + c, work, field, col, lane, part % 4);
 }
 
 // Stage-0 inputs of a grid row's inverse from its P and Q.
@@ -199,19 +243,27 @@ __device__ __forceinline__ void load_pair(const cf32* __restrict__ p, cf32 (&v)[
 }
 
 template <class G>
-__global__ void __launch_bounds__(G::PR::kThreads) ns_rows_kernel(cf32* work, long long pairs)
+__global__ void __launch_bounds__(G::PR::kThreads)
+    ns_rows_kernel(const cf32* __restrict__ work, cf32* __restrict__ bins, int fields, bool by_xcd)
 {
     using P = typename G::PR;
     constexpr int RL = P::template radix<P::kStages - 1>();
     __shared__ cf32 lds[G::kRowLds];
     const int lane = static_cast<int>(threadIdx.x) % P::L;
     const int t = static_cast<int>(threadIdx.x) / P::L;
-    const long long pair = static_cast<long long>(blockIdx.x) * P::T + t;
+    const auto [field, part] = block_of<G::kRowParts, 1>(by_xcd);
+    const long long pairs = static_cast<long long>(fields) * (G::N / 2);
+    const long long pair = G::kRowParts > 1
+                               ? static_cast<long long>(field) * (G::N / 2) + part * P::T + t
+                               : static_cast<long long>(blockIdx.x) * P::T + t;
+    if (pair - t >= pairs) {
+        return;  // the whole workgroup
+    }
     cf32* const s = lds + t * P::kStride;
     const bool live = pair < pairs;
     // Lane groups past the end repeat the last pair and store nothing.
-    cf32* const row0 = work + (live ? pair : pairs - 1) * (2LL * 4 * G::kPitch);
-    cf32* const row1 = row0 + 4 * G::kPitch;
+    const cf32* const row0 = work + (live ? pair : pairs - 1) * (2LL * 4 * G::kPitch);
+    const cf32* const row1 = row0 + 4 * G::kPitch;
     cf32 g[P::E];  // both rows' products, in the forward's input slots
 #pragma unroll
     for (int y = 0; y < 2; ++y) {
@@ -243,71 +295,140 @@ __global__ void __launch_bounds__(G::PR::kThreads) ns_rows_kernel(cf32* work, lo
     if (live) {
         // G = G0 + i G1 of two real rows: G0[k] = (G[k] + conj G[-k]) / 2 and
         // G1[k] = (G[k] - conj G[-k]) / 2i.
+        cf32* const out = bins + pair * (2LL * G::kPitch);
         for (int k = lane; k < G::kW; k += P::L) {
             const cf32 f = s[pad(k)];
             const cf32 h = s[pad((G::N - k) & (G::N - 1))];
-            row0[k] = cf32{0.5f * (f.re + h.re), 0.5f * (f.im - h.im)};
-            row1[k] = cf32{0.5f * (f.im + h.im), 0.5f * (h.re - f.re)};
+            out[k] = cf32{0.5f * (f.re + h.re), 0.5f * (f.im - h.im)};
+            out[G::kPitch + k] = cf32{0.5f * (f.im + h.im), 0.5f * (h.re - f.re)};
         }
     }
 }
 
-// One tile of kT columns: the forward column transforms and the update of the kept rows. out_f and
-// out_w may be w0 or f0 (each lane reads the elements it is about to write), so none is restrict.
-template <class G>
-__global__ void __launch_bounds__(G::kColumnThreads)
-    ns_update_kernel(const cf32* __restrict__ work, const cf32* w0, const cf32* f0, cf32* out_f,
-                     cf32* out_w, const cf32* __restrict__ forcing_hat,
-                     const float* __restrict__ nu, int nu_stride, float drag, float dt, int stage)
+// What a stage's update reads and writes. The stores of stage 0 go to out_f, those of stage 1 to
+// out_w.
+struct NsUpdate {
+    const cf32* bins;
+    const cf32* w0;
+    const cf32* f0;
+    cf32* out_f;
+    cf32* out_w;
+    const cf32* forcing_hat;
+    const float* nu;
+    int nu_stride;
+    float drag;
+    float dt;
+};
+
+// One tile of kT columns: the forward column transforms of the rows' bins and the update. v: the
+// state that the stage arrives at, element lane + (e / RL) L + (e % RL) N / RL in slot e, zeros where
+// the layout keeps no row. Every load comes before the first store, which may alias w0.
+template <class G, int Stage>
+__device__ __forceinline__ void update_columns(cf32 (&v)[G::PC::E], cf32* s, const NsUpdate& a,
+                                               int field, int col, int lane, bool store)
 {
     using P = typename G::PC;
     using Lay = PaddedRows<G::kT>;
     constexpr int R0 = P::template radix<0>();
     constexpr int RL = P::template radix<P::kStages - 1>();
-    __shared__ cf32 s[G::kColumnLds];
-    const int field = static_cast<int>(blockIdx.x) / G::kTiles;
-    const int tid = threadIdx.x;
-    const int c = tid % G::kT;
-    const int lane = tid / G::kT;
-    const int col = (static_cast<int>(blockIdx.x) % G::kTiles) * G::kT + c;
-    const cf32* const in = work + static_cast<long long>(field) * G::N * 4 * G::kPitch + col;
-    const float nu_f = nu[static_cast<long long>(field) * nu_stride];
-    cf32 v[P::E];
+    const cf32* const in = a.bins + static_cast<long long>(field) * G::N * G::kPitch + col;
+    const float nu_f = a.nu[static_cast<long long>(field) * a.nu_stride];
     const bool live = col < G::kW;
 #pragma unroll
     for (int e = 0; e < P::E; ++e) {
         const int y = input_index<P, 0>(lane, e / R0, e % R0);
-        v[e] = live ? in[y * (4 * G::kPitch)] : czero();
-    }
-    run_stages<P, 0, false, false, Lay>(v, s + c, lane, nullptr);
-    if (!live) {
-        return;  // past the last barrier
+        v[e] = live ? in[y * G::kPitch] : czero();
     }
     const long long base = static_cast<long long>(field) * G::kRows * G::kW;
+    const auto row_of = [lane](int e) {
+        return lane + (e / RL) * P::L + (e % RL) * (P::N / RL);
+    };
+    run_stages<P, 0, false, false, Lay>(v, s, lane, nullptr);
+    cf32 w[P::E];
+    cf32 f[P::E];
+    cf32 forcing[P::E];
+#pragma unroll
+    for (int e = 0; e < P::E; ++e) {
+        const int r = state_row<G>(row_of(e));
+        const bool has = live && r >= 0;
+        const int at = has ? r * G::kW + col : 0;
+        w[e] = has ? a.w0[base + at] : czero();
+        forcing[e] = has ? a.forcing_hat[at] : czero();
+        if constexpr (Stage == 1) {
+            f[e] = has ? a.f0[base + at] : czero();
+        }
+    }
     const float kmax = static_cast<float>(G::N) / 3.0f;
     const float kx = static_cast<float>(col);
+#pragma unroll
+    for (int e = 0; e < P::E; ++e) {
+        const int i = row_of(e);
+        const int r = state_row<G>(i);
+        const float ky = ky_of<G>(i);
+        const bool kept = kx <= kmax && fabsf(ky) <= kmax;
+        const cf32 F = csub(forcing[e], kept ? v[e] : czero());
+        const float linear = -nu_f * (kx * kx + ky * ky) - a.drag;
+        const float ex = 1.0f + 0.5f * a.dt * linear;
+        const float im = reciprocal(1.0f - 0.5f * a.dt * linear);
+        const cf32 add = Stage == 0 ? cscale(F, a.dt) : cscale(cadd(f[e], F), 0.5f * a.dt);
+        const cf32 next = cscale(cadd(cscale(w[e], ex), add), im);
+        const bool has = live && r >= 0;
+        if (has && store) {
+            (Stage == 0 ? a.out_f : a.out_w)[base + r * G::kW + col] = Stage == 0 ? F : next;
+        }
+        v[e] = has ? next : czero();
+    }
+}
+
+// The last stage of a call.
+template <class G>
+__global__ void __launch_bounds__(G::kColumnThreads)
+    ns_update_kernel(NsUpdate a, int fields, bool by_xcd)
+{
+    __shared__ cf32 s[G::kColumnLds];
+    const auto [field, part] = block_of<G::kTiles, 1>(by_xcd);
+    if (field >= fields) {
+        return;  // the whole workgroup
+    }
+    const int c = static_cast<int>(threadIdx.x) % G::kT;
+    const int col = part * G::kT + c;
+    cf32 v[G::PC::E];
+    update_columns<G, 1>(v, s + c, a, field, col, static_cast<int>(threadIdx.x) / G::kT, true);
+}
+
+// The update of a stage and the derived columns of the next one, Sets of a tile's four per workgroup.
+// The workgroups of a tile each form its new state, which one of them stores.
+template <class G, int Stage, int Sets>
+__global__ void __launch_bounds__(G::kColumnThreads)
+    ns_update_columns_kernel(NsUpdate a, cf32* __restrict__ work, int fields, bool by_xcd)
+{
+    using P = typename G::PC;
+    __shared__ cf32 s[G::kColumnLds];
+    constexpr int kShare = 4 / Sets;
+    const auto [field, part] = block_of<kShare * G::kTiles, kShare>(by_xcd);
+    const int first = part % kShare * Sets;
+    if (field >= fields) {
+        return;  // the whole workgroup
+    }
+    const int c = static_cast<int>(threadIdx.x) % G::kT;
+    const int lane = static_cast<int>(threadIdx.x) / G::kT;
+    const int col = part / kShare * G::kT + c;
+    cf32 state[P::E];
+    update_columns<G, Stage>(state, s + c, a, field, col, lane, first == 0);
+    cf32 next[P::E];  // in the inverse's input slots
     static_for<0, P::E>([&](auto ei) {
         constexpr int e = decltype(ei)::value;
-        const int i = lane + (e / RL) * P::L + (e % RL) * (P::N / RL);
-        const int r = state_row<G>(i);
-        if (r >= 0) {
-            const int at = r * G::kW + col;
-            const float ky = ky_of<G>(i);
-            const bool kept = kx <= kmax && fabsf(ky) <= kmax;
-            const cf32 F = csub(forcing_hat[at], kept ? v[e] : czero());
-            const float linear = -nu_f * (kx * kx + ky * ky) - drag;
-            const float ex = 1.0f + 0.5f * dt * linear;
-            const float im = reciprocal(1.0f - 0.5f * dt * linear);
-            const cf32 w = w0[base + at];
-            if (stage == 0) {
-                out_f[base + at] = F;
-                out_w[base + at] = cscale(cadd(cscale(w, ex), cscale(F, dt)), im);
-            } else {
-                const cf32 sum = cadd(f0[base + at], F);
-                out_w[base + at] = cscale(cadd(cscale(w, ex), cscale(sum, 0.5f * dt)), im);
-            }
-        }
+        next[forward_slot_of<P>(e)] = state[e];
     });
+#pragma unroll
+    for (int set = 0; set < Sets; ++set) {
+        cf32 v[P::E];
+#pragma unroll
+        for (int e = 0; e < P::E; ++e) {
+            v[e] = next[e];
+        }
+        derived_columns<G>(v, s + c, work, field, col, lane, first + set);
+    }
 }
 
 struct NsArrays {
@@ -321,24 +442,55 @@ struct NsArrays {
     float dt;
 };
 
+// Whether a field's blocks all run on one XCD, so that what one kernel writes is in the L2 the next
+// one reads it from. Always up to 256^2 (six steps, best of either order: one field of 128^2 in the
+// full layout 186 -> 146 us, nine 209 -> 170, one field of 256^2 164 -> 155, 48 357 -> 334). Larger
+// fields do not fit an L2, and an idle XCD costs more: only if at most an eighth of the XCDs are
+// idle (512^2: one field 222 against 299 us, 12 fields 404 against 414, 8 fields 331 -> 322, 30 797
+// -> 722; 1024^2: four fields 542 against 880 us, 8 fields 981 -> 899).
 template <class G>
-void stage(const NsArrays& a, const cf32* state, const cf32* w0, const cf32* f0, cf32* out_f,
-           cf32* out_w, cf32* spectra, const float* nu, int fields, int which, hipStream_t stream)
+bool by_xcd(int fields)
 {
-    const int items = fields * G::kTiles;
-    const unsigned column_blocks = static_cast<unsigned>((items + 7) / 8) * 32u;
-    hipLaunchKernelGGL(ns_columns_kernel<G>, dim3(column_blocks), dim3(G::kColumnThreads), 0,
-                       stream, state, spectra, items);
+    const int rounds = (fields + 7) / 8;
+    return G::N <= 256 || fields >= 7 * rounds;
+}
+
+template <class G>
+void launch_rows(const cf32* spectra, cf32* bins, int fields, hipStream_t stream)
+{
+    const int pairs = fields * (G::N / 2);
+    const unsigned blocks = G::kRowParts > 1 ? blocks_of<G::kRowParts, 1>(fields, by_xcd<G>(fields))
+                                             : static_cast<unsigned>((pairs + G::PR::T - 1) / G::PR::T);
+    hipLaunchKernelGGL(ns_rows_kernel<G>, dim3(blocks), dim3(G::PR::kThreads), 0, stream, spectra,
+                       bins, fields, by_xcd<G>(fields));
     SPX_LAUNCH_CHECK();
-    const long long pairs = static_cast<long long>(fields) * (G::N / 2);
-    const auto row_blocks = static_cast<unsigned>((pairs + G::PR::T - 1) / G::PR::T);
-    hipLaunchKernelGGL(ns_rows_kernel<G>, dim3(row_blocks), dim3(G::PR::kThreads), 0, stream,
-                       spectra, pairs);
+}
+
+template <class G, int Stage, int Sets>
+void launch_update_columns(const NsUpdate& a, cf32* spectra, int fields, hipStream_t stream)
+{
+    const unsigned blocks = blocks_of<4 / Sets * G::kTiles, 4 / Sets>(fields, by_xcd<G>(fields));
+    hipLaunchKernelGGL((ns_update_columns_kernel<G, Stage, Sets>), dim3(blocks),
+                       dim3(G::kColumnThreads), 0, stream, a, spectra, fields, by_xcd<G>(fields));
     SPX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(ns_update_kernel<G>, dim3(static_cast<unsigned>(items)),
-                       dim3(G::kColumnThreads), 0, stream, spectra, w0, f0, out_f, out_w,
-                       a.forcing_hat, nu, a.nu_stride, a.drag, a.dt, which);
-    SPX_LAUNCH_CHECK();
+}
+
+// One, two or all four sets per workgroup: the fewest workgroups that repeat a tile's update while
+// there are at most two waves per SIMD of the chip. 256^2 pruned, six steps with 1 / 2 / 4 sets:
+// 8 fields 169 / 167 / 185 us, 16 fields 199 / 195 / 200, 48 fields 377 / 339 / 334, 100 fields
+// 641 / 559 / 547; 1024^2: one field 368 / 394 / 451, two 447 / 401 / 457, four 618 / 632 / 542.
+template <class G, int Stage>
+void update_and_columns(const NsUpdate& a, cf32* spectra, int fields, hipStream_t stream)
+{
+    const long long waves = static_cast<long long>(fields) * G::kTiles * (G::kColumnThreads / 64);
+    const long long filled = 8LL * device_cus();
+    if (4 * waves <= filled) {
+        launch_update_columns<G, Stage, 1>(a, spectra, fields, stream);
+    } else if (2 * waves <= filled) {
+        launch_update_columns<G, Stage, 2>(a, spectra, fields, stream);
+    } else {
+        launch_update_columns<G, Stage, 4>(a, spectra, fields, stream);
+    }
 }
 
 // Fields advanced together: as many as keep the derived spectra (the array that every kernel
@@ -354,7 +506,7 @@ template <class G>
 std::size_t workspace(int batch)
 {
     const int group = std::min(batch, fields_per_group<G>());
-    return static_cast<std::size_t>(group) * (4 * G::N * G::kPitch + 2 * G::kRows * G::kW);
+    return static_cast<std::size_t>(group) * (5 * G::N * G::kPitch + 2 * G::kRows * G::kW);
 }
 
 template <class G>
@@ -363,21 +515,36 @@ void advance(const NsArrays& a, int batch, int steps, hipStream_t stream)
     constexpr long long kField = static_cast<long long>(G::kRows) * G::kW;
     const int most = std::min(batch, fields_per_group<G>());
     const int groups = (batch + most - 1) / most;
+    constexpr long long kGrid = static_cast<long long>(G::N) * G::kPitch;
     cf32* const spectra = a.work;
-    cf32* const tendency = spectra + static_cast<long long>(most) * 4 * G::N * G::kPitch;
-    cf32* const predicted = tendency + most * kField;
+    cf32* const bins = spectra + most * 4 * kGrid;
+    cf32* const tendency = bins + most * kGrid;
+    cf32* const spare = tendency + most * kField;
     for (int g = 0; g < groups; ++g) {
         // Even shares, so that no group is left with a few fields.
         const int first = static_cast<int>(static_cast<long long>(batch) * g / groups);
         const int fields = static_cast<int>(static_cast<long long>(batch) * (g + 1) / groups) - first;
         cf32* const out = a.w_out + first * kField;
-        const float* const nu = a.nu + static_cast<long long>(first) * a.nu_stride;
-        const cf32* w = a.w_in + first * kField;
+        NsUpdate u{bins, a.w_in + first * kField, tendency, tendency, nullptr, a.forcing_hat,
+                   a.nu + static_cast<long long>(first) * a.nu_stride, a.nu_stride, a.drag, a.dt};
+        hipLaunchKernelGGL(ns_columns_kernel<G>, dim3(blocks_of<4 * G::kTiles, 4>(fields, by_xcd<G>(fields))),
+                           dim3(G::kColumnThreads), 0, stream, u.w0, spectra, fields, by_xcd<G>(fields));
+        SPX_LAUNCH_CHECK();
         for (int s = 0; s < steps; ++s) {
-            stage<G>(a, w, w, nullptr, tendency, predicted, spectra, nu, fields, 0, stream);
-            stage<G>(a, predicted, w, tendency, nullptr, out, spectra, nu, fields, 1, stream);
-            w = out;
+            launch_rows<G>(spectra, bins, fields, stream);
+            update_and_columns<G, 0>(u, spectra, fields, stream);
+            launch_rows<G>(spectra, bins, fields, stream);
+            if (s + 1 < steps) {
+                // Not into w0, which other workgroups of the tile still read.
+                u.out_w = u.w0 == spare ? out : spare;
+                update_and_columns<G, 1>(u, spectra, fields, stream);
+                u.w0 = u.out_w;
+            }
         }
+        u.out_w = out;
+        hipLaunchKernelGGL(ns_update_kernel<G>, dim3(blocks_of<G::kTiles, 1>(fields, by_xcd<G>(fields))),
+                           dim3(G::kColumnThreads), 0, stream, u, fields, by_xcd<G>(fields));
+        SPX_LAUNCH_CHECK();
     }
 }
 

@@ -24,9 +24,9 @@ simulate() use between frames, runs k steps as one launch. The single stages are
 requires it, False never.
 
 Where it does not apply (other grids from 32 to 1024, and the full layout) and fused is None, a
-Stockham fft_impl's step() and advance() run each stage as three kernels
-(torch.ops.spectral.ns_advance_grid): inverse columns of the derived fields, rows with the product,
-forward columns with the update. fused=False keeps the transforms and elementwise operations
+Stockham fft_impl's step() and advance() run each stage as two kernels
+(torch.ops.spectral.ns_advance_grid): rows with the product, then forward columns with the update
+and the inverse columns of the next stage's derived fields. fused=False keeps the transforms and elementwise operations
 apart.
 """
 
@@ -136,7 +136,7 @@ class GpuSolver:
                 f"(got pruned={pruned}, fft_impl='{fft_impl}', n={n})"
             )
         self.fused = fusable if fused is None else bool(fused)
-        # step() and advance() by the three-kernel stages, unless fused=False asks for the composed
+        # step() and advance() by the grid stages, unless fused=False asks for the composed
         # transforms, drag or dt broadcasts, or a subclass brings its own step.
         self._grid_steps = (fused is None and not fusable and fft_impl.startswith("stockham")
                             and _C.ns_grid_supports(n)
@@ -206,7 +206,7 @@ class GpuSolver:
         return w_hat
 
     def _takes_grid_steps(self, w_hat: torch.Tensor) -> bool:
-        """Whether the three-kernel stages give what the composed step gives for this state: a
+        """Whether the grid stages give what the composed step gives for this state: a
         complex64 state of this layout on the solver's device that needs no gradient, with one
         viscosity or one per field of exactly its batch shape (others broadcast)."""
         if not self._grid_steps:

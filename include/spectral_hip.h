@@ -174,8 +174,8 @@ int spx_ns_steps(const void* w_in, void* w_out, void* work, const void* forcing_
                  const float* nu, int nu_stride, float drag, float dt, int n, int batch,
                  int steps, hipStream_t stream);
 
-/* spx_ns_grid_steps: the same steps for the grids and layouts without a one-workgroup kernel, three
- * launches per stage: n a power of two from 32 to 1024 (spx_ns_grid_supports), the pruned layout
+/* spx_ns_grid_steps: the same steps for the grids and layouts without a one-workgroup kernel, two
+ * launches per stage and one more each for a call's start and end: n a power of two from 32 to 1024 (spx_ns_grid_supports), the pruned layout
  * above or (pruned = 0) the rfft2 layout, n x (n/2 + 1) values per field. `steps` >= 1 steps of
  * w_in into w_out, which are the same array or do not overlap; `work` holds
  * spx_ns_grid_workspace complex values and overlaps no other array. forcing_hat: one field's

@@ -240,7 +240,7 @@ def test_frames_take_the_many_step_path(rng):
         assert torch.equal(got, want)
 
 
-# The three-kernel stages (torch.ops.spectral.ns_advance_grid, C ABI spx_ns_grid_steps), which step()
+# The grid stages (torch.ops.spectral.ns_advance_grid, C ABI spx_ns_grid_steps), which step()
 # and advance() take on grids and layouts without a one-workgroup kernel: against the composed step.
 
 
@@ -268,6 +268,26 @@ def test_grid_steps_match_the_composed_step(rng, n, batch, pruned):
             expected = composed.step(expected)
             assert relative(advance(w, steps), expected) < 3e-6, f"{steps} steps"
         assert torch.equal(w, kept)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pruned", [True, False], ids=["pruned", "full"])
+@pytest.mark.parametrize("n, batch", [(64, 90), (64, 180), (128, 26), (128, 55), (256, 12),
+                                      (256, 25), (512, 6), (512, 8), (512, 13), (512, 15),
+                                      (1024, 2), (1024, 4), (1024, 7)])
+def test_grid_steps_share_a_tile_among_workgroups(rng, n, batch, pruned):
+    # Two and four of a tile's derived columns per workgroup, with a field's workgroups on one XCD
+    # or over all of them.
+    flow, dt = Flow(viscosity=rng.uniform(1e-3, 5e-3, batch), drag=0.1), 1e-3
+    solver = GpuSolver(n, flow, dt, pruned=pruned)
+    composed = GpuSolver(n, flow, dt, pruned=pruned, fused=False)
+    w = random_state(rng, n, (batch,), composed)
+    expected = w
+    for steps in (1, 2, 3):
+        expected = composed.step(expected)
+        got = torch.ops.spectral.ns_advance_grid(w, solver.forcing_hat, solver.nu, 0.1, dt, n,
+                                                 steps, pruned)
+        assert relative(got, expected) < 3e-6, f"{steps} steps"  # two float32 orders, as above
 
 
 @pytest.mark.gpu
