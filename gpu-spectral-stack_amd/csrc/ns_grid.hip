@@ -29,11 +29,12 @@
 //
 // Measured on MI355X (256^2 pruned, 48 fields, six steps and a frame): 434 us with the update and
 // the columns apart (10.3 and 12.8 us; rows 13.0 us), 349 us as here (rows 13.0, update and
-// columns 17 us a launch). The update and columns are
-// bound by their instructions (about 1700 per wave, 44 waves per field), the rows by theirs and the
-// LDS exchanges; about 4 us of each launch is its ramp and drain. Rows with the second row's loads
-// ahead of the first row's transforms were 1.7 us slower (registers), with one row per lane group
-// 4 us slower (the pair's forward then runs on both).
+// columns 17 us a launch). Both kernels issue vector instructions for 6 us of a launch and wait on
+// loads and exchanges for the rest, two to three waves per SIMD; 4 us of each launch is its ramp
+// and drain. More and shorter waves (4 values per lane) were 8 % slower at 48 fields and 8 % faster
+// at eight; fewer and longer ones (16 values) 3 % slower. Rows with the second row's loads ahead of
+// the first row's transforms were 1.7 us slower (registers), with one row per lane group 4 us
+// slower (the pair's forward then runs on both).
 
 #include "stockham.hpp"
 
