@@ -31,8 +31,7 @@
 // the columns apart (10.3 and 12.8 us; rows 13.0 us), 349 us as here (rows 13.0, update and
 // columns 17 us a launch). Both kernels issue vector instructions for 6 us of a launch and wait on
 // loads and exchanges for the rest, two to three waves per SIMD; 4 us of each launch is its ramp
-// and drain. More and shorter waves (4 values per lane) were 8 % slower at 48 fields and 8 % faster
-// at eight; fewer and longer ones (16 values) 3 % slower. Rows with the second row's loads ahead of
+// and drain. Rows with the second row's loads ahead of
 // the first row's transforms were 1.7 us slower (registers), with one row per lane group 4 us
 // slower (the pair's forward then runs on both).
 
@@ -55,7 +54,8 @@ struct ColumnPlan : Plan<N, R, E> {
     static constexpr bool kWaveLocal = false;
 };
 
-template <int N_, bool Pruned_>
+// Few: few fields of 256^2, which take 4 values per lane, twice the waves, each half as long.
+template <int N_, bool Pruned_, bool Few = false>
 struct NsGrid {
     static constexpr int N = N_;
     static constexpr bool kPruned = Pruned_;
@@ -70,15 +70,16 @@ struct NsGrid {
     static constexpr int kTiles = (kW + kT - 1) / kT;
     // Radix and values per lane of the columns: 8 while a tile then takes at most 512 lanes. At 256
     // the update waits on its loads, not on its stages: 12.4 us with 16 values, 10.3 us with 8.
-    static constexpr int kR = N <= 256 ? 8 : 16;
+    static constexpr int kR = Few ? 4 : N <= 256 ? 8 : 16;
     using PC = ColumnPlan<N, kR, kR>;
     static constexpr int kColumnThreads = kT * PC::L;
     static constexpr int kColumnLds = pad(N - 1) * kT + kT;
-    static constexpr int kRE = N <= 512 ? 8 : 16;          // rows: one wave or less per transform
+    static constexpr int kRE = Few ? 4 : N <= 512 ? 8 : 16;          // rows: one wave or less per transform
     using PR = Plan<N, kRE, kRE>;
     static constexpr int kRowParts = cmax(1, N / 2 / PR::T);  // row workgroups per field
     static constexpr int kRowLds = PR::T * PR::kStride;
 
+    static_assert(!Few || N == 256, "the shape measured");
     static_assert(PR::L <= 64 && kColumnThreads <= 1024, "workgroup shapes");
     static_assert(slots_match<PR>() && slots_match<PC>(),
                   "one direction's outputs must be the other's inputs");
@@ -549,9 +550,12 @@ void advance(const NsArrays& a, int batch, int steps, hipStream_t stream)
     }
 }
 
-// f.template operator()<G>() for the kernels' grid of this size and layout.
+// f(G{}) for the kernels' grid of this size, layout and number of fields. Up to 16 fields of 256^2
+// (two per XCD) leave SIMDs without a wave, and shorter waves are then faster: six steps, 8 / 4
+// values per lane, one field 160 -> 146 us, 8 fields 168 -> 152 (204 -> 190 in the full layout), 16
+// fields 194 -> 191, 33 fields 284 -> 311.
 template <class F>
-auto dispatch(int n, bool pruned, F&& f)
+auto dispatch(int n, bool pruned, int batch, F&& f)
 {
     const auto layout = [&](auto size) {
         constexpr int N = decltype(size)::value;
@@ -561,7 +565,11 @@ auto dispatch(int n, bool pruned, F&& f)
     case 32: return layout(std::integral_constant<int, 32>{});
     case 64: return layout(std::integral_constant<int, 64>{});
     case 128: return layout(std::integral_constant<int, 128>{});
-    case 256: return layout(std::integral_constant<int, 256>{});
+    case 256:
+        if (batch <= 16) {
+            return pruned ? f(NsGrid<256, true, true>{}) : f(NsGrid<256, false, true>{});
+        }
+        return layout(std::integral_constant<int, 256>{});
     case 512: return layout(std::integral_constant<int, 512>{});
     case 1024: return layout(std::integral_constant<int, 1024>{});
     default:
@@ -581,7 +589,7 @@ std::size_t ns_grid_workspace(int n, bool pruned, int batch)
         throw InvalidArgument("ns_grid_workspace: need batch >= 1");
     }
     return dev::dispatch(
-        n, pruned, [&](auto g) { return dev::workspace<decltype(g)>(batch); });
+        n, pruned, batch, [&](auto g) { return dev::workspace<decltype(g)>(batch); });
 }
 
 void ns_grid_steps(const cf32* w_in, cf32* w_out, cf32* work, const cf32* forcing_hat,
@@ -597,7 +605,7 @@ void ns_grid_steps(const cf32* w_in, cf32* w_out, cf32* work, const cf32* forcin
             "ns_grid_steps: w_in, w_out, work, forcing_hat and nu must not be null");
     }
     const dev::NsArrays arrays{w_in, w_out, work, forcing_hat, nu, nu_stride, drag, dt};
-    dev::dispatch(n, pruned,
+    dev::dispatch(n, pruned, batch,
                   [&](auto g) { dev::advance<decltype(g)>(arrays, batch, steps, stream); });
 }
 

@@ -272,8 +272,8 @@ def test_grid_steps_match_the_composed_step(rng, n, batch, pruned):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("pruned", [True, False], ids=["pruned", "full"])
-@pytest.mark.parametrize("n, batch", [(64, 90), (64, 180), (128, 26), (128, 55), (256, 12),
-                                      (256, 25), (512, 6), (512, 8), (512, 13), (512, 15),
+@pytest.mark.parametrize("n, batch", [(64, 90), (64, 180), (128, 26), (128, 55), (256, 1),
+                                      (256, 4), (256, 12), (256, 16), (256, 17), (256, 25), (512, 6), (512, 8), (512, 13), (512, 15),
                                       (1024, 2), (1024, 4), (1024, 7)])
 def test_grid_steps_share_a_tile_among_workgroups(rng, n, batch, pruned):
     # Two and four of a tile's derived columns per workgroup, with a field's workgroups on one XCD
