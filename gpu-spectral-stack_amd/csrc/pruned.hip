@@ -8,7 +8,11 @@
 //
 //   SinglePass   one kernel per array, the tile in LDS (fft2_fused.hpp / fft2_modes.hpp)
 //   InKernel     pruned real rows that write only m2 columns, then pruned columns that keep
-//                only the 2 m1 rows (the inverse mirrored), through an n1 x m2 workspace
+//                only the 2 m1 rows (the inverse mirrored), through an n1 x m2 workspace. Shapes
+//                beyond SinglePass whose kept columns alone fit the LDS run as one kernel too, from
+//                a number of arrays on (Fused2dFns::modes_supports), if input and output lie apart.
+//                Their workspace is the two passes' whatever the batch: one sized for the largest
+//                batch then serves every smaller one, and a call over its own input still runs.
 //   Transposes   implementations without pruned kernels (naive): the mode selection is folded
 //                into the transposes of the transpose method. Forward: real rows (n1 x w), a
 //                transpose that keeps only the m2 kept columns (m2 x n1), the column transforms
@@ -26,6 +30,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cstdint>
 
 namespace spx {
 namespace {
@@ -58,6 +63,7 @@ struct ModesPlan {
     std::size_t full;    // n1 x w per array: the real rows' output (Transposes)
     std::size_t narrow;  // n1 x m2 per array: the kept columns
     std::size_t real;    // scratch of the generic real rows
+    bool narrow_tiles;   // InKernel: one kernel if input and output lie apart
 
     std::size_t words() const
     {
@@ -88,19 +94,39 @@ ModesPlan plan_modes(const FftImpl& impl, int n1, int n2, int m1, int m2, int ba
     expect(batch >= 1 && static_cast<long long>(batch) * std::max(n1, n2) <= INT_MAX,
            [] { return std::string("rfft2 modes: batch out of range"); });
 
-    ModesPlan p{ModesRoute::Transposes, n1, n2, m1, m2, batch, n2 / 2 + 1, 0, 0, 0};
+    ModesPlan p{ModesRoute::Transposes, n1, n2, m1, m2, batch, n2 / 2 + 1, 0, 0, 0, false};
     p.narrow = values(n1, m2, batch);
-    if (impl.fused != nullptr
-        && (impl.fused->supports(n1, n2)
-            || impl.fused->modes_supports(n1, n2, m1, m2, batch))) {
+    if (impl.fused != nullptr && impl.fused->supports(n1, n2)) {
         p.route = ModesRoute::SinglePass;
     } else if (impl.pruned != nullptr) {
         p.route = ModesRoute::InKernel;
+        p.narrow_tiles =
+            impl.fused != nullptr && impl.fused->modes_supports(n1, n2, m1, m2, batch);
     } else {
         p.full = values(n1, p.w, batch);
         p.real = impl.real_needs_work ? values(n1, n2 / 2, batch) : 0;
     }
     return p;
+}
+
+// Whether the request runs as one kernel, for these arrays.
+bool one_kernel(const ModesPlan& p, const float* real, const cf32* modes)
+{
+    if (p.route == ModesRoute::SinglePass) {
+        return true;
+    }
+    const auto r = reinterpret_cast<std::uintptr_t>(real);
+    const auto c = reinterpret_cast<std::uintptr_t>(modes);
+    return p.narrow_tiles && (r + values(p.n1, p.n2, p.batch) * sizeof(float) <= c
+                              || c + values(2 * p.m1, p.m2, p.batch) * sizeof(cf32) <= r);
+}
+
+void expect_workspace(const ModesPlan& p, const cf32* work)
+{
+    expect(work != nullptr, [&] {
+        return "rfft2 modes: this request needs a workspace of "
+               + str(static_cast<long long>(p.words())) + " complex values";
+    });
 }
 
 void check_1d(const FftImpl& impl, int n, int keep, int batch)
@@ -200,10 +226,11 @@ void rfft2_modes(const FftImpl& impl, const float* x, cf32* modes, int n1, int n
                  int m2, int batch, cf32* work, hipStream_t stream)
 {
     const ModesPlan p = plan_modes(impl, n1, n2, m1, m2, batch);
-    if (p.route == ModesRoute::SinglePass) {
+    if (one_kernel(p, x, modes)) {
         impl.fused->r2c(x, modes, n1, n2, m1, m2, batch, stream);
         return;
     }
+    expect_workspace(p, work);
     if (p.route == ModesRoute::InKernel) {
         impl.pruned->r2c_work(x, work, n2, batch * n1, m2, stream);  // n1 x m2 per array
         impl.pruned->columns(work, modes, n1, m2, batch, 0, m1, Direction::Forward, stream);
@@ -230,10 +257,11 @@ void irfft2_modes(const FftImpl& impl, const cf32* modes, float* y, int n1, int 
                   int m2, int batch, cf32* work, hipStream_t stream)
 {
     const ModesPlan p = plan_modes(impl, n1, n2, m1, m2, batch);
-    if (p.route == ModesRoute::SinglePass) {
+    if (one_kernel(p, y, modes)) {
         impl.fused->c2r(modes, y, n1, n2, m1, m2, batch, stream);
         return;
     }
+    expect_workspace(p, work);
     if (p.route == ModesRoute::InKernel) {
         impl.pruned->columns_work(modes, work, n1, m2, batch, m1, 0, Direction::Inverse, stream);
         impl.pruned->c2r(work, y, n2, batch * n1, m2, stream);  // columns m2.. are zero

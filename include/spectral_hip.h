@@ -130,6 +130,8 @@ int spx_transpose(const void* x, void* y, int rows, int cols, int batch, hipStre
  * fft_c2c_pruned: forward (batch, n) -> (batch, keep); inverse (batch, keep) -> (batch, n).
  * rfft2_modes: (batch, n1, n2) real -> (batch, 2 m1, m2) modes, rows 0 .. m1-1 then
  *      n1-m1 .. n1-1 of rfft2, columns 0 .. m2-1. irfft2_modes is its inverse (other modes 0).
+ *      The workspace queries never shrink as the batch grows: `work` sized for the largest batch
+ *      serves the smaller ones. A call that needs a workspace refuses a NULL one.
  * gather_modes / scatter_modes copy those modes out of / into full n1 x w arrays (m1 = 0: all
  *      n1 rows); scatter zeroes `full` first. */
 int spx_fft_c2c_pruned_workspace(int impl, int n, int keep, int batch, size_t* count);

@@ -449,6 +449,58 @@ def test_direct_columns_over_many_tiles(lib, rng, n, slabs):
     assert_transform_close(back, _fft_columns(padded, True), n, axes=(-2,))
 
 
+@pytest.mark.parametrize("impl", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize(("n1", "n2"), [(64, 64), (128, 128), (128, 256), (256, 128), (256, 256),
+                                        (256, 512), (512, 512)])
+def test_modes_workspace_grows_with_the_batch(lib, impl, n1, n2):
+    # Queries are host arithmetic, so these need no GPU: a workspace sized for the largest batch
+    # serves every smaller one, and a request that needs one refuses NULL.
+    count = ctypes.c_size_t()
+    p, q = ctypes.c_void_p(1 << 40), ctypes.c_void_p(1 << 41)
+    for query, call in ((lib.spx_rfft2_modes_workspace, lib.spx_rfft2_modes),
+                        (lib.spx_irfft2_modes_workspace, lib.spx_irfft2_modes)):
+        for m2 in (1, n2 // 16, n2 // 8, n2 // 8 + 1):
+            last = 0
+            for batch in (1, 2, 40, 47, 48, 49, 64, 100, 256):
+                assert query(impl, n1, n2, 8, m2, batch, ctypes.byref(count)) == SPX_OK
+                assert count.value >= last, (m2, batch)
+                last = count.value
+        if last > 0:
+            assert call(impl, p, q, n1, n2, 8, n2 // 8 + 1, 4, None, None) == SPX_EINVAL
+            assert "needs a workspace" in _last(lib)
+            if (n1, n2) == (256, 256):
+                assert call(impl, p, q, n1, n2, 8, 32, 40, None, None) == SPX_EINVAL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(("n1", "n2", "batch"), [(128, 256, 3), (256, 128, 3), (256, 256, 47),
+                                                 (256, 256, 48)])
+def test_pruned_transforms_over_their_own_input(lib, rng, n1, n2, batch):
+    # The modes written over the field they come from and back: the two-pass route's order allows
+    # it, at sizes that run as one kernel when the arrays lie apart.
+    from oracle.tolerance import random_real
+
+    m1, m2 = 16, 16
+    count = ctypes.c_size_t()
+    assert lib.spx_rfft2_modes_workspace(3, n1, n2, m1, m2, batch, ctypes.byref(count)) == SPX_OK
+    work = torch.empty(count.value, dtype=torch.complex64, device="cuda")
+    field = torch.from_numpy(random_real(rng, (batch, n1, n2))).cuda()
+    modes = torch.empty(batch, 2 * m1, m2, dtype=torch.complex64, device="cuda")
+    back = torch.empty_like(field)
+    shape = (n1, n2, m1, m2, batch, _ptr(work), None)
+    assert lib.spx_rfft2_modes(3, _ptr(field), _ptr(modes), *shape) == SPX_OK
+    assert lib.spx_irfft2_modes(3, _ptr(modes), _ptr(back), *shape) == SPX_OK
+    assert lib.spx_rfft2_modes(3, _ptr(field), _ptr(field), *shape) == SPX_OK
+    torch.cuda.synchronize()
+    over = torch.view_as_complex(field.view(-1)[: 2 * modes.numel()].view(-1, 2)).view_as(modes)
+    # Two float32 transforms of 2^15 and 2^16 points: each about 3e-7 off, in the 2-norm.
+    assert torch.linalg.vector_norm(over - modes) < 2e-6 * torch.linalg.vector_norm(modes)
+    field.view(-1)[: 2 * modes.numel()] = torch.view_as_real(modes).reshape(-1)
+    assert lib.spx_irfft2_modes(3, _ptr(field), _ptr(field), *shape) == SPX_OK
+    torch.cuda.synchronize()
+    assert torch.linalg.vector_norm(field - back) < 2e-6 * torch.linalg.vector_norm(back)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("inverse", [0, 1])
 @pytest.mark.parametrize(("n", "cols", "slabs"), [(1024, 16, 63), (1024, 16, 64), (1024, 17, 61),
