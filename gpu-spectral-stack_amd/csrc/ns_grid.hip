@@ -581,6 +581,23 @@ auto dispatch(int n, bool pruned, int batch, F&& f)
 }  // namespace
 }  // namespace dev
 
+namespace {
+
+// An array in memory.
+struct Span {
+    const void* first;
+    std::uintptr_t bytes;
+
+    bool overlaps(const Span& other) const
+    {
+        const auto a = reinterpret_cast<std::uintptr_t>(first);
+        const auto b = reinterpret_cast<std::uintptr_t>(other.first);
+        return a < b + other.bytes && b < a + bytes;
+    }
+};
+
+}  // namespace
+
 bool ns_grid_supports(int n) { return is_pow2(n) && n >= 32 && n <= 1024; }
 
 std::size_t ns_grid_workspace(int n, bool pruned, int batch)
@@ -605,8 +622,23 @@ void ns_grid_steps(const cf32* w_in, cf32* w_out, cf32* work, const cf32* forcin
             "ns_grid_steps: w_in, w_out, work, forcing_hat and nu must not be null");
     }
     const dev::NsArrays arrays{w_in, w_out, work, forcing_hat, nu, nu_stride, drag, dt};
-    dev::dispatch(n, pruned, batch,
-                  [&](auto g) { dev::advance<decltype(g)>(arrays, batch, steps, stream); });
+    dev::dispatch(n, pruned, batch, [&](auto g) {
+        using G = decltype(g);
+        constexpr std::uintptr_t kField = sizeof(cf32) * G::kRows * G::kW;
+        const Span in{w_in, batch * kField};
+        const Span out{w_out, batch * kField};
+        const Span wk{work, dev::workspace<G>(batch) * sizeof(cf32)};
+        const Span forcing{forcing_hat, kField};
+        const Span nus{nu, (nu_stride == 0 ? 1 : batch) * sizeof(float)};
+        if (wk.overlaps(in) || wk.overlaps(out) || wk.overlaps(forcing) || wk.overlaps(nus)) {
+            throw InvalidArgument("ns_grid_steps: work must not overlap another array");
+        }
+        if (w_in != w_out && in.overlaps(out)) {
+            throw InvalidArgument(
+                "ns_grid_steps: w_in and w_out must be the same array or not overlap");
+        }
+        dev::advance<G>(arrays, batch, steps, stream);
+    });
 }
 
 }  // namespace spx

@@ -156,6 +156,73 @@ def test_navier_stokes_steps_arguments(lib):
     assert steps(wk=state + field, count=0) == SPX_OK
 
 
+@pytest.mark.parametrize(("n", "pruned", "batch"), [(32, 1, 1), (32, 0, 3), (256, 1, 16),
+                                                    (256, 1, 17), (1024, 0, 9)])
+def test_navier_stokes_grid_steps_arguments(lib, n, pruned, batch):
+    # Every refusal comes before anything is queued, so these need no GPU.
+    f, v = ctypes.c_float, ctypes.c_void_p
+    rows, cols = (2 * (n // 3 + 1), n // 3 + 1) if pruned else (n, n // 2 + 1)
+    count = ctypes.c_size_t()
+    assert lib.spx_ns_grid_workspace(n, pruned, batch, ctypes.byref(count)) == SPX_OK
+    state_bytes, work_bytes = 8 * batch * rows * cols, 8 * count.value
+    state, work, forcing, nu = 1 << 40, 1 << 42, 1 << 43, 1 << 44
+
+    def steps(n=n, batch=batch, count=1, nu_stride=1, w_in=state, w_out=state, wk=work):
+        return lib.spx_ns_grid_steps(v(w_in), v(w_out), v(wk), v(forcing), v(nu), nu_stride,
+                                     f(0.1), f(1e-3), n, pruned, batch, count, None)
+
+    assert steps(n=16) == SPX_EINVAL and "32 to 1024" in _last(lib)
+    assert steps(n=96) == SPX_EINVAL and steps(n=2048) == SPX_EINVAL
+    assert steps(batch=0) == SPX_EINVAL and "batch >= 1" in _last(lib)
+    assert steps(count=0) == SPX_EINVAL and "steps >= 1" in _last(lib)
+    assert steps(nu_stride=2) == SPX_EINVAL and "nu_stride 0 or 1" in _last(lib)
+    assert steps(wk=None) == SPX_EINVAL and "must not be null" in _last(lib)
+    assert steps(w_in=None) == SPX_EINVAL and steps(w_out=None) == SPX_EINVAL
+    # The work area's end reaching into the state, the forcing and the viscosities, the state's end
+    # into the work area, and the work area over a separate output.
+    for wk in (state, state - work_bytes + 8, state + state_bytes - 8, forcing - work_bytes + 8,
+               nu - work_bytes + 4, nu + 4 * batch - 4):
+        assert steps(wk=wk) == SPX_EINVAL and "work must not overlap" in _last(lib)
+    assert steps(w_out=work + work_bytes - 8) == SPX_EINVAL
+    # Input and output: the same array, or apart; a partial overlap is refused.
+    for w_out in (state + 8, state - 8, state + state_bytes - 8):
+        assert steps(w_out=w_out) == SPX_EINVAL and "the same array" in _last(lib)
+    assert lib.spx_ns_grid_workspace(n, pruned, 0, ctypes.byref(count)) == SPX_EINVAL
+    assert lib.spx_ns_grid_workspace(48, pruned, 1, ctypes.byref(count)) == SPX_EINVAL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(("n", "pruned", "batch"), [(32, 1, 5), (256, 1, 3), (256, 1, 20),
+                                                    (1024, 1, 12), (1024, 0, 8)])
+def test_navier_stokes_grid_steps_in_place(lib, rng, n, pruned, batch):
+    # In place against out of place, bit for bit, at every turn of the two state arrays; nothing
+    # is written past the queried workspace. The 1024^2 batches are one field more than a group
+    # (11 pruned, 7 in the full layout), so they run as two groups.
+    from spectral.flow import Flow
+    from spectral.flow.gpu import GpuSolver
+
+    solver = GpuSolver(n, Flow(viscosity=np.linspace(1e-3, 4e-3, batch)), 1e-3,
+                       pruned=bool(pruned), fused=False)
+    w = solver.to_spectral(torch.from_numpy(rng.standard_normal((batch, n, n))).float().cuda())
+    kept = w.clone()
+    count = ctypes.c_size_t()
+    assert lib.spx_ns_grid_workspace(n, pruned, batch, ctypes.byref(count)) == SPX_OK
+    work = torch.full((count.value + 64,), 7.0, dtype=torch.complex64, device="cuda")
+    args = (_ptr(work), _ptr(solver.forcing_hat), _ptr(solver.nu), 1, ctypes.c_float(0.1),
+            ctypes.c_float(1e-3), n, pruned, batch)
+    before = w
+    for steps in (1, 2, 3):
+        out, over = torch.full_like(w, float("nan")), w.clone()
+        assert lib.spx_ns_grid_steps(_ptr(w), _ptr(out), *args, steps, None) == SPX_OK
+        assert lib.spx_ns_grid_steps(_ptr(over), _ptr(over), *args, steps, None) == SPX_OK
+        torch.cuda.synchronize()
+        assert torch.equal(w, kept) and torch.equal(out, over), f"{steps} steps"
+        before = solver.step(before)
+        error = torch.linalg.vector_norm(out - before) / torch.linalg.vector_norm(before)
+        assert float(error) < 3e-6, f"{steps} steps"  # two float32 orders, 5e-7 each
+    assert bool((work[count.value:] == 7.0).all())
+
+
 def test_workspace_queries(lib):
     count = ctypes.c_size_t()
     assert lib.spx_fft2_c2c_workspace(3, 1, 8, 8, 2, ctypes.byref(count)) == SPX_OK
