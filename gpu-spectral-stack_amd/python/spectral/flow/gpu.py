@@ -26,8 +26,11 @@ requires it, False never.
 Where it does not apply (other grids from 32 to 1024, and the full layout) and fused is None, a
 Stockham fft_impl's step() and advance() run each stage as two kernels
 (torch.ops.spectral.ns_advance_grid): rows with the product, then forward columns with the update
-and the inverse columns of the next stage's derived fields. fused=False keeps the transforms and elementwise operations
-apart.
+and the inverse columns of the next stage's derived fields. Those kernels form the operators
+themselves, so a solver whose explicit, implicit, derivatives, nu, dt, spectral (mask, transforms),
+step or tendency has been replaced or edited in place since its constructor takes the composed step,
+which reads them; so does a step being captured into a graph, whose replays are to read what these
+tensors hold by then. fused=False keeps the transforms and elementwise operations apart.
 """
 
 from __future__ import annotations
@@ -116,6 +119,8 @@ class Spectral:
 class GpuSolver:
     """Advances a batch of vorticity fields; viscosity a float or one value per trajectory."""
 
+    # Ordinary tensors whatever the caller's mode: inference tensors count no versions.
+    @torch.inference_mode(False)
     def __init__(
         self,
         n: int,
@@ -137,12 +142,10 @@ class GpuSolver:
             )
         self.fused = fusable if fused is None else bool(fused)
         # step() and advance() by the grid stages, unless fused=False asks for the composed
-        # transforms, drag or dt broadcasts, or a subclass brings its own step.
+        # transforms or drag or dt broadcasts; per call, _takes_grid_steps decides.
         self._grid_steps = (fused is None and not fusable and fft_impl.startswith("stockham")
                             and _C.ns_grid_supports(n)
-                            and isinstance(flow.drag, (int, float)) and isinstance(dt, (int, float))
-                            and type(self).step is GpuSolver.step
-                            and type(self).tendency is GpuSolver.tendency)
+                            and isinstance(flow.drag, (int, float)) and isinstance(dt, (int, float)))
 
         k2 = s.kx**2 + s.ky**2
         over_k2 = torch.where(k2 > 0, 1.0 / k2.clamp(min=1.0), torch.zeros_like(k2))
@@ -162,6 +165,8 @@ class GpuSolver:
         half_l = 0.5 * dt * (-per_field * k2 - flow.drag)
         self.explicit = (1.0 + half_l).to(torch.complex64)
         self.implicit = (1.0 / (1.0 - half_l)).to(torch.complex64)
+        if self._grid_steps:
+            self._drag, self._built = flow.drag, self._formula()
 
     def to_spectral(self, w: torch.Tensor) -> torch.Tensor:
         """omega_hat of physical vorticity (..., n, n), projected onto the dealiased modes."""
@@ -199,23 +204,46 @@ class GpuSolver:
                 steps)
         if steps > 0 and self._takes_grid_steps(w_hat):
             return torch.ops.spectral.ns_advance_grid.default(
-                w_hat, self.forcing_hat, self.nu, float(self.flow.drag), float(self.dt), self.n,
-                steps, self.spectral.pruned)
+                w_hat, self.forcing_hat, self.nu, float(self._drag), float(self.dt), self.n, steps,
+                self.spectral.pruned)
         for _ in range(steps):
             w_hat = self.step(w_hat)
         return w_hat
 
+    def _formula(self) -> tuple[tuple, tuple]:
+        """What a composed step is made of besides the state and the forcing: objects, compared by
+        identity (this solver holds them), and values."""
+        s = self.spectral
+        tensors = (self.explicit, self.implicit, self.derivatives, self.nu, s.mask)
+        methods = (type(self).step, type(self).tendency, type(s).forward, type(s).inverse)
+        own = (vars(self).get("step"), vars(self).get("tendency"), vars(s).get("forward"),
+               vars(s).get("inverse"))
+        objects = (*methods, *own, s, s._forward, s._inverse, *tensors)
+        edits = tuple(None if t.is_inference() else t._version for t in tensors)
+        return objects, (self.n, self.dt if isinstance(self.dt, (int, float)) else None, *edits)
+
     def _takes_grid_steps(self, w_hat: torch.Tensor) -> bool:
         """Whether the grid stages give what the composed step gives for this state: a
-        complex64 state of this layout on the solver's device that needs no gradient, with one
-        viscosity or one per field of exactly its batch shape (others broadcast)."""
+        complex64 state of this layout on the solver's device, with one viscosity or one per field
+        of exactly its batch shape (others broadcast), nothing that needs a gradient, the operators
+        as the constructor made them, and no graph being captured."""
         if not self._grid_steps:
             return False
+        objects, values = self._formula()
+        forcing = self.forcing_hat
         nu_shape, lead = self.explicit.shape[:-2], w_hat.shape[:-2]
         return (w_hat.dtype == torch.complex64 and w_hat.device == self.nu.device
-                and w_hat.numel() > 0 and w_hat.shape[-2:] == self.forcing_hat.shape
+                and w_hat.numel() > 0 and w_hat.shape[-2:] == forcing.shape
+                and forcing.dtype == torch.complex64 and forcing.device == w_hat.device
                 and (nu_shape == lead or (self.nu.numel() == 1 and len(nu_shape) <= len(lead)))
-                and not (w_hat.requires_grad and torch.is_grad_enabled()))
+                and values == self._built[1]
+                and all(now is then for now, then in zip(objects, self._built[0]))
+                and objects[: len(_METHODS)] == _METHODS
+                and not (torch.is_grad_enabled()
+                         and any(t.requires_grad for t in (w_hat, forcing, self.explicit,
+                                                           self.implicit, self.derivatives,
+                                                           self.spectral.mask)))
+                and not torch.cuda.is_current_stream_capturing())
 
     def frames(self, w0: torch.Tensor, steps: int, record_every: int = 1) -> Iterator[torch.Tensor]:
         """Physical vorticity at step 0 (the dealiased initial condition) and after every
@@ -232,3 +260,7 @@ class GpuSolver:
     def simulate(self, w0: torch.Tensor, steps: int, record_every: int = 1) -> torch.Tensor:
         """Every frame of frames(), stacked: (frames, ..., n, n)."""
         return torch.stack(list(self.frames(w0, steps, record_every)))
+
+
+# What the grid stages compute; a subclass or a patch that brings its own is composed.
+_METHODS = (GpuSolver.step, GpuSolver.tendency, Spectral.forward, Spectral.inverse)

@@ -323,3 +323,126 @@ def test_grid_steps_leave_other_states_to_the_composed_step(rng):
         torch.ops.spectral.ns_advance_grid(w, shared.forcing_hat, shared.nu, 0.1, dt, 16, 1, True)
     with pytest.raises(RuntimeError, match="steps must be >= 1"):
         torch.ops.spectral.ns_advance_grid(w, shared.forcing_hat, shared.nu, 0.1, dt, n, 0, False)
+
+
+def _replaced(name, change):
+    return lambda solver: setattr(solver, name, change(getattr(solver, name)))
+
+
+def _in_place(name, change):
+    return lambda solver: change(getattr(solver, name))
+
+
+def _hyperviscous(solver):
+    solver.explicit, solver.implicit = solver.explicit * 0.9, solver.implicit * 0.9
+
+
+def _smaller_mask(solver):
+    solver.spectral.mask[:, 5:] = 0.0
+
+
+def _no_advection(solver):
+    solver.tendency = lambda w_hat: solver.forcing_hat - 0.1 * w_hat
+
+
+def _half_products(solver):
+    forward = solver.spectral.forward
+    solver.spectral.forward = lambda x: 0.5 * forward(x)
+
+
+SOLVER_EDITS = {
+    "explicit and implicit replaced": _hyperviscous,
+    "implicit in place": _in_place("implicit", lambda t: t.mul_(0.9)),
+    "explicit through a view": _in_place("explicit", lambda t: t[..., 3:, :].zero_()),
+    "derivatives in place": _in_place("derivatives", lambda t: t[2].zero_()),
+    "another mask": _smaller_mask,
+    "mask replaced": lambda solver: setattr(solver.spectral, "mask", 0.5 * solver.spectral.mask),
+    "another dt": _replaced("dt", lambda dt: 0.5 * dt),
+    "tendency on the instance": _no_advection,
+    "a transform on the instance": _half_products,
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pruned", [True, False], ids=["pruned", "full"])
+@pytest.mark.parametrize("edit", SOLVER_EDITS.values(), ids=SOLVER_EDITS.keys())
+@pytest.mark.parametrize("mode", [torch.no_grad, torch.inference_mode], ids=["plain", "inference"])
+def test_grid_steps_honour_an_edited_solver(rng, edit, pruned, mode):
+    # The kernels form the operators themselves; an edited solver must step by its own.
+    n, dt = 32, 0.2
+    flow = Flow(viscosity=2e-2, drag=0.1)
+    with mode():
+        solver = GpuSolver(n, flow, dt, pruned=pruned)
+        composed = GpuSolver(n, flow, dt, pruned=pruned, fused=False)
+        w = random_state(rng, n, (3,), composed)
+        before = solver.advance(w, 2)
+        assert solver._takes_grid_steps(w)
+        edit(solver)
+        edit(composed)
+        assert not solver._takes_grid_steps(w)
+        expected = composed.step(composed.step(w))
+        assert torch.equal(solver.advance(w, 2), expected)
+        assert torch.equal(solver.step(solver.step(w)), expected)
+        assert relative(before, expected) > 1e-3
+
+
+@pytest.mark.gpu
+def test_grid_steps_keep_the_constructors_drag(rng):
+    # The composed step never reads the flow again; neither do the grid stages.
+    flow = Flow(viscosity=2e-3, drag=0.1)
+    solver = GpuSolver(32, flow, 1e-3)
+    w = random_state(rng, 32, (2,), solver)
+    expected = solver.step(w)
+    solver.flow = Flow(viscosity=2e-3, drag=5.0)
+    assert solver._takes_grid_steps(w) and torch.equal(solver.step(w), expected)
+
+
+@pytest.mark.gpu
+def test_grid_steps_leave_gradients_to_the_composed_step(rng):
+    solver = GpuSolver(32, Flow(viscosity=2e-3), 1e-3)
+    w = random_state(rng, 32, (2,), solver)
+    for tensor in (solver.forcing_hat, solver.explicit, solver.spectral.mask):
+        assert solver._takes_grid_steps(w)
+        tensor.requires_grad_()
+        assert not solver._takes_grid_steps(w)
+        with torch.no_grad():
+            assert solver._takes_grid_steps(w)
+        tensor.requires_grad_(False)
+
+
+@pytest.mark.gpu
+def test_grid_steps_honour_a_patched_class(rng, monkeypatch):
+    solver = GpuSolver(32, Flow(viscosity=2e-3), 1e-3)
+    w = random_state(rng, 32, (2,), solver)
+    assert solver._takes_grid_steps(w)
+    monkeypatch.setattr(GpuSolver, "tendency", lambda self, w_hat: torch.zeros_like(w_hat))
+    assert not solver._takes_grid_steps(w)
+    assert not GpuSolver(32, Flow(viscosity=2e-3), 1e-3)._takes_grid_steps(w)
+
+
+@pytest.mark.gpu
+def test_a_captured_step_reads_the_operators_at_replay(rng):
+    # 256^2 eager steps are grid stages; a captured one is composed, so an operator updated in place
+    # between replays counts.
+    solver = GpuSolver(256, Flow(viscosity=2e-3), 1e-3, pruned=True)
+    w = random_state(rng, 256, (2,), solver)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        solver.step(w)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = solver.step(w)
+    graph.replay()
+    eager = solver.step(w)
+    torch.cuda.synchronize()
+    assert relative(out, eager) < 3e-6  # two float32 orders of the same sums
+    for factor in (0.9, 0.8, 0.7):
+        solver.implicit.mul_(factor)
+        graph.replay()
+        expected = solver.step(w)
+        torch.cuda.synchronize()
+        assert torch.equal(out, expected), f"implicit x {factor}"
+        assert relative(expected, eager) > 0.05
