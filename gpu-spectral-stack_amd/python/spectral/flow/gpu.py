@@ -184,8 +184,10 @@ class GpuSolver:
         return self.forcing_hat - self.spectral.forward(product) * self.spectral.mask
 
     def step(self, w_hat: torch.Tensor) -> torch.Tensor:
-        if self.fused or self._takes_grid_steps(w_hat):
+        if self.fused:
             return self.advance(w_hat, 1)
+        if self._takes_grid_steps(w_hat):
+            return self._grid_advance(w_hat, 1)
         carried = self.explicit * w_hat
         f0 = self.tendency(w_hat)
         predicted = (carried + self.dt * f0) * self.implicit
@@ -203,12 +205,15 @@ class GpuSolver:
                 w_hat, self.forcing_hat, self.nu, float(self.flow.drag), float(self.dt), self.n,
                 steps)
         if steps > 0 and self._takes_grid_steps(w_hat):
-            return torch.ops.spectral.ns_advance_grid.default(
-                w_hat, self.forcing_hat, self.nu, float(self._drag), float(self.dt), self.n, steps,
-                self.spectral.pruned)
+            return self._grid_advance(w_hat, steps)
         for _ in range(steps):
             w_hat = self.step(w_hat)
         return w_hat
+
+    def _grid_advance(self, w_hat: torch.Tensor, steps: int) -> torch.Tensor:
+        return torch.ops.spectral.ns_advance_grid.default(
+            w_hat, self.forcing_hat, self.nu, float(self._drag), float(self.dt), self.n, steps,
+            self.spectral.pruned)
 
     def _formula(self) -> tuple[tuple, tuple]:
         """What a composed step is made of besides the state and the forcing: objects, compared by

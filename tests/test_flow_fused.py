@@ -446,3 +446,22 @@ def test_a_captured_step_reads_the_operators_at_replay(rng):
         torch.cuda.synchronize()
         assert torch.equal(out, expected), f"implicit x {factor}"
         assert relative(expected, eager) > 0.05
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n, pruned", [(32, True), (128, False)])
+def test_a_subclass_may_build_advance_on_step(rng, n, pruned):
+    class Counting(GpuSolver):
+        count = 0
+
+        def advance(self, w_hat, steps):
+            for _ in range(steps):
+                w_hat = self.step(w_hat)
+                self.count += 1
+            return w_hat
+
+    solver = Counting(n, Flow(viscosity=2e-3), 1e-3, pruned=pruned)
+    w = random_state(rng, n, (2,), solver)
+    plain = GpuSolver(n, Flow(viscosity=2e-3), 1e-3, pruned=pruned)
+    expected = plain.step(plain.step(plain.step(w)))
+    assert torch.equal(solver.advance(w, 3), expected) and solver.count == 3
