@@ -23,6 +23,7 @@ Files are gpu-rf-pipeline's: .cf32 interleaved little-endian float32 I/Q, .f32 r
 from __future__ import annotations
 
 import argparse
+import functools
 import sys
 from pathlib import Path
 
@@ -35,6 +36,7 @@ TORCH_BACKENDS: tuple[str, ...] = ("rocfft", "cufft")
 FFT_BACKENDS: tuple[str, ...] = (*TORCH_BACKENDS, *ops.FFT_IMPLS)
 WINDOWS: tuple[str, ...] = ("rect", "hann", "hamming", "blackman")
 FUSED_MAX_NFFT = 16384  # the longest frame or block the one-launch paths take
+_DIRECT_TAPS = _C.rf_fir_direct_taps()  # the longest filter rf_fir_direct takes
 
 # Each window as a generalized cosine sum w[k] = sum_j (-1)^j a_j cos(2 pi j k / n), periodic
 # (scipy.signal.get_window's fftbins=True convention).
@@ -131,6 +133,7 @@ def spectrum(
     return fft(frames(x, nfft) * w, fft_impl=fft_impl)
 
 
+@functools.lru_cache(maxsize=1024, typed=True)
 def default_nfft(num_taps: int) -> int:
     """fir()'s block size for a filter of num_taps taps: the power of two nearest above four
     times the length, at least 64 and at most 4096, unless the filter alone needs more (then the
@@ -142,13 +145,26 @@ def default_nfft(num_taps: int) -> int:
     return nfft if nfft <= 4096 else max(4096, above(num_taps))
 
 
-def _summed_directly(taps: torch.Tensor, samples: int) -> bool:
-    """Whether fir() without a given block size runs as the convolution sum (one launch on the matrix
-    cores, no filter spectrum) instead of overlap-save blocks. The sum's work grows with the taps: at
-    2^22 samples it takes 18.2 us for 63 taps and 21 us for 95, blocks 22.1 and 19.6 us; up to 2^20
-    samples it takes 6 to 9 us for as many as it supports, blocks 12 us."""
-    longest = _C.rf_fir_direct_taps() if samples <= 1 << 20 else 64
-    return not taps.is_complex() and taps.numel() <= longest
+@functools.lru_cache(maxsize=1024)
+def _summed_directly(taps: int, n: int, samples: int, nfft: int) -> bool:
+    """Whether fir() of `samples` samples in rows of n, without a given block size, runs as the
+    convolution sum (one launch on the matrix cores, no filter spectrum) instead of overlap-save
+    blocks of nfft; up to 64 taps, or as many as the sum supports up to 2^20 samples (its work grows
+    with the taps: at 2^22 samples it takes 17.2 us for 63 taps and 21 us for 95, blocks 20.0 and 19.2
+    us; up to 2^20 samples 7 to 8 us, blocks 12.8 us).
+
+    Its work also grows with the rows: each runs whole steps of 1024 outputs, a quarter of
+    3 + 2 ceil((taps + 15) / 16) ns apiece on the whole GPU (65536 rows of 16: 113 us for 15 taps,
+    211 for 63), where a block costs about 1.1 us per 2^20 points beyond the two launches' 12.8 us
+    (12.8 and 31.8 us). So steps worth 9 us at most (4096 rows of 64 or 256: 10.0 / 11.9 / 13.9 us
+    for 15 / 31 / 48 taps), or fewer than the blocks' points pay for: at 96 points to a quarter ns
+    the two are equal (8192 rows of 512, 31 taps: 24.0 and 24.3 us; 2048 rows of 1536: 16.5 and 17.3
+    us for 48 taps, 18.0 and 17.1 for 63)."""
+    rows = samples // max(n, 1)
+    quarters = rows * _ceil_div(n, 1024) * (3 + 2 * _ceil_div(taps + 15, 16))
+    if quarters <= 36864:
+        return True
+    return 96 * quarters <= rows * _ceil_div(n, nfft - taps + 1) * nfft
 
 
 def _taps_spectrum(taps: torch.Tensor, nfft: int, fft_impl: str, device) -> torch.Tensor:
@@ -180,7 +196,9 @@ def fir(
     nfft = nfft if block_given else default_nfft(m)
     if nfft < m or nfft & (nfft - 1):
         raise ValueError(f"nfft must be a power of two of at least len(taps) = {m}, got {nfft}")
-    if not block_given and fft_impl.startswith("stockham") and _summed_directly(taps, x.numel()):
+    if (m <= _DIRECT_TAPS and not block_given and fft_impl.startswith("stockham")
+            and (m <= 64 or x.numel() <= 1 << 20) and not taps.is_complex() and x.dim() > 0
+            and _summed_directly(m, x.size(-1), x.numel(), nfft)):
         return torch.ops.spectral.rf_fir_direct.default(x, taps.to(x.device, torch.float32))
     h = _taps_spectrum(taps, nfft, fft_impl, x.device)
     if _one_launch(fft_impl, nfft):

@@ -421,3 +421,45 @@ def test_short_real_filters_keep_the_calls_rules(rng):
         torch.ops.spectral.rf_fir_direct(x, torch.ones(130, device="cuda"))
     with pytest.raises(ValueError, match="float32"):
         torch.ops.spectral.rf_fir_direct(x, h.cuda())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(("shape", "taps", "direct"), [
+    ((1 << 14,), 63, True), ((1 << 22,), 63, True), ((1 << 20,), 129, True),
+    ((1 << 20,), 130, False), (((1 << 20) + 1,), 65, False),
+    ((1024, 64), 129, True), ((64, 16384), 112, True), ((2048, 2048), 63, True),
+    # Rows shorter than a step of 1024 outputs: few of them, then so many that the steps' work
+    # outweighs the blocks'.
+    ((4096, 64), 31, True), ((4096, 64), 48, False), ((16384, 64), 15, False),
+    ((65536, 16), 15, False), ((65536, 16), 63, False), ((16384, 256), 31, False),
+    ((8192, 512), 15, True), ((8192, 512), 48, False), ((4096, 1025), 48, False),
+])
+def test_short_real_filters_take_the_cheaper_route(rng, monkeypatch, shape, taps, direct):
+    x = torch.zeros(shape, dtype=torch.complex64, device="cuda")
+    x[..., : 1 + shape[-1] // 2] = 1.0 - 0.5j
+    h = torch.from_numpy(rng.standard_normal(taps).astype(np.float32))
+    summed = torch.ops.spectral.rf_fir_direct
+    calls = []
+
+    class Spy:
+        @staticmethod
+        def default(*args):
+            calls.append(args)
+            return summed.default(*args)
+
+    monkeypatch.setattr(torch.ops.spectral, "rf_fir_direct", Spy)
+    y = rf.fir(x, h, fft_impl="stockham_r8")
+    assert bool(calls) == direct
+    expected = scipy.signal.lfilter(h.double().numpy(), 1.0, x.view(-1, shape[-1])[0].cpu().numpy())
+    got = y.view(-1, shape[-1])[-1].cpu().numpy()
+    assert np.abs(got - expected).max() <= taps * 2.4e-7 * np.abs(h.numpy()).sum() * 1.2 + 1e-5
+
+
+@pytest.mark.gpu
+def test_empty_recordings_filter_to_empty_ones():
+    h = torch.ones(5)
+    for shape in ((0,), (0, 7), (3, 0)):
+        x = torch.zeros(shape, dtype=torch.complex64, device="cuda")
+        assert rf.fir(x, h, fft_impl="stockham_r8").shape == shape
+    with pytest.raises(RuntimeError, match="at least one dimension"):
+        rf.fir(torch.zeros((), dtype=torch.complex64, device="cuda"), h, fft_impl="stockham_r8")
