@@ -33,7 +33,11 @@ struct SplitColumnPlan : SplitPlan<N> {
 // the slabs' columns laid end to end. An exchange row holds one float of each column, with a spare
 // row after every 16 (PaddedRows): the four rows that a wave's 64 lanes touch lie on four distinct
 // quarters of the 64 banks. Consecutive tiles, which share lines when a row of the arrays is no
-// multiple of 16 values, run on one XCD.
+// multiple of 16 values, run on one XCD, and the loads leave those lines in its L2 (nontemporal
+// loads: 1024 x 33 out of place, 528 tiles, 76.6 against 64 us; whole lines 1 % slower too). Fewer than
+// 256 tiles of 1024-point columns in place keep the hint (fft2 of 32 arrays of 1024 x 64, 128 tiles,
+// 22.5 against 23.2 us, of 96 of 1024 x 32, 192 tiles, 24.8 against 26.0; 256 tiles 34.3 against 33.3,
+// 512 49.7 against 44.7).
 template <class P, bool Inv, bool Table>
 __global__ void __launch_bounds__(P::kLanes, P::kWavesPerSimd)
     columns_split_kernel(StridedIo io, long long batch, const cf32* table)
@@ -50,12 +54,13 @@ __global__ void __launch_bounds__(P::kLanes, P::kWavesPerSimd)
     const long long slab = (live ? t : batch - 1) / io.cols;
     const long long at = slab * P::N * io.cols + ((live ? t : batch - 1) - slab * io.cols)
                          + static_cast<long long>(lane) * io.cols;
+    const bool once = P::N == 1024 && io.stream_out && io.x == io.y && gridDim.x < 256;
     cf32 v[P::E];
     const cf32* const src = io.x + at;
     static_for<0, P::E>([&](auto ei) {
         constexpr int e = decltype(ei)::value;
         constexpr long long off = (e / R0) * P::L + (e % R0) * (P::N / R0);
-        v[e] = io.stream_out ? ld_stream(src + off * io.cols) : src[off * io.cols];
+        v[e] = once ? ld_stream(src + off * io.cols) : src[off * io.cols];
     });
     run_stages_split<P, 0, Inv, Table, Lay>(v, s + c, lane, table);
     if (live) {

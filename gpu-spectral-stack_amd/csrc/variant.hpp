@@ -186,18 +186,46 @@ inline constexpr bool kFusedPersistent = SPX_FUSED_PERSISTENT != 0;
 #endif
 inline constexpr bool kPersistentLarge = SPX_LARGE_PERSISTENT != 0;
 
-// Unpruned columns of 1024 and 2048 points, radix-8 variants: tiles of 16 columns in registers
-// (fft_split.hpp). At 1024 points from 64 tiles on: the persistent kernel's 8-column tiles are twice
-// as many and less work each, and keep the small batches (2 tiles 15.3 against 13.7 us for an
-// rfft2; 64 tiles 14.5 against 14.2 us; 256 tiles 16.2 against 21.4 us; 1024 tiles, 2^24 points,
-// 58.7 against 69.9 us). At 2048 points wherever the columns ran as two passes: 2048 x 64 arrays,
-// fft2, one 29.3 -> 20.2 us, 64 of them 72.5 -> 53.5 us.
+// Whether unpruned columns of 1024 or 2048 points run as tiles of 16 columns in registers
+// (fft_split.hpp; radix-8 variants). Figures: the time of the kernel otherwise run over this one's,
+// on 256 compute units.
+//
+// 1024 points, against the persistent kernel's tiles of 8 columns: twice as many and half as long,
+// they keep the batches that leave compute units idle. Out of place 64 tiles 0.87-0.92, 96
+// 0.92-1.08, 128 1.03-1.24 (plain stores of 64 columns and more 0.98: rfft2 of 8 arrays of 1024 x
+// 512), 136 1.09-1.33, 192 1.2-1.5, 1024 1.13-1.4. In place the two halves of a line are written by
+// two of its workgroups, and these tiles win from 64 on (fft2 of 16 arrays of 1024 x 64 1.14, of 32
+// 1.2), narrow matrices near its 256 workgroups excepted (32 columns, fft2: 64 tiles 1.05, 96 1.14,
+// 120 0.96, 128 1.3; 16 columns, 128 tiles 0.97). Where rows are no whole lines (columns no multiple
+// of 16) either kernel shares lines: out of place 1.04-1.37 from 256 tiles, 0.8-1.1 below; in place
+// 0.6-1.4 without order.
+//
+// 2048 points, against two passes (long_columns): 1.2-1.9, whatever the number of tiles; with shared
+// lines out of place 1.0-1.2 up to 64 tiles and 0.7-1.0 beyond, in place 0.96-1.2 up to 16.
 template <int N, int R>
 bool split_columns(const StridedIo& io, long long batch)
 {
+    static_assert(N == 1024 || N == 2048, "the lengths measured");
     if constexpr (R == 8 && kRadix16) {
-        return io.m1_in == 0 && io.m1_out == 0 && io.cols >= (N == 1024 ? 16 : 32)
-               && batch >= (N == 1024 ? 64 : 1) * SplitColumnPlan<N>::kTile;
+        constexpr int T = SplitColumnPlan<N>::kTile;
+        const bool whole_lines = io.cols % 16 == 0;
+        const bool in_place = io.x == io.y;
+        if (io.m1_in > 0 || io.m1_out > 0 || io.cols < 16) {
+            return false;
+        }
+        if constexpr (N == 2048) {
+            return io.cols >= 32 && (whole_lines || batch <= (in_place ? 16 : 64) * T);
+        }
+        if (!whole_lines) {
+            return !in_place && batch >= 256 * T;
+        }
+        if (in_place) {
+            return batch >= 136 * T
+                   || (batch >= 64 * T
+                       && (io.cols >= 64
+                           || (io.cols >= 32 && (batch <= 112 * T || batch >= 128 * T))));
+        }
+        return batch >= (io.stream_out || io.cols < 64 ? 128 : 136) * T;
     }
     return false;
 }
@@ -875,8 +903,8 @@ struct Stockham {
         launch_rows<n2>(rows, inverse, static_cast<long long>(batch) * n1, stream);
     }
 
-    // Columns of n = 2048 (without kSplit) or 4096 points as two passes of 64 x (n / 64) (a four-step split of
-    // the column axis): a single pass would stage only 4 or 2 columns per workgroup, reading
+    // Columns of n = 2048 (where not split_columns) or 4096 points as two passes of 64 x (n / 64) (a
+    // four-step split of the column axis): a single pass would stage only 4 or 2 columns per workgroup, reading
     // runs of 32 or 16 bytes; each of these passes stages 32 columns of 64 points (256-byte
     // runs). Pass A runs
     // the 64-point transforms over rows j1 (n/64) + j2 and twiddles them (x -> work); pass B runs
@@ -948,7 +976,11 @@ struct Stockham {
             throw InvalidArgument("stockham columns: a pruned transform cannot run in place");
         }
         const long long batch = static_cast<long long>(cols) * slabs;
-        if (n >= 2048 && m1_in == 0 && m1_out == 0 && cols >= 32 && !(kSplit && n == 2048)) {
+        const bool inverse = direction == Direction::Inverse;
+        const float scale = inverse ? 1.0f / static_cast<float>(n) : 1.0f;
+        const dev::StridedIo io{x, y, cols, scale, m1_in, m1_out, stream_out};
+        if (n >= 2048 && m1_in == 0 && m1_out == 0 && cols >= 32
+            && !(n == 2048 && dev::split_columns<2048, R>(io, batch))) {
             long_columns(x, y, n, cols, slabs, direction, stream, stream_out);
             return;
         }
@@ -959,9 +991,6 @@ struct Stockham {
             }
             return;
         }
-        const bool inverse = direction == Direction::Inverse;
-        const float scale = inverse ? 1.0f / static_cast<float>(n) : 1.0f;
-        const dev::StridedIo io{x, y, cols, scale, m1_in, m1_out, stream_out};
         if (inverse) {
             dev::dispatch_strided_columns<R, true, Table>(n, io, batch, stream);
         } else {

@@ -592,6 +592,33 @@ def test_long_columns_in_register_tiles(lib, rng, n, cols, slabs, inverse):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("impl", [3, 4])
+@pytest.mark.parametrize(("n", "cols", "slabs"), [
+    (1024, 16, 127), (1024, 16, 128), (1024, 16, 136), (1024, 32, 31), (1024, 32, 32), (1024, 32, 57),
+    (1024, 32, 64), (1024, 64, 16),
+    (1024, 64, 33), (1024, 80, 28), (1024, 17, 240), (1024, 17, 241), (1024, 513, 8),
+    (2048, 33, 7), (2048, 33, 8), (2048, 33, 31), (2048, 33, 32), (2048, 48, 40), (2048, 1025, 1)])
+def test_long_columns_at_both_sides_of_the_rule(lib, rng, impl, n, cols, slabs):
+    # Tiles of 16 columns in registers, or the kernels they replace: by the number of tiles, whole or
+    # shared lines, in place or not.
+    from oracle.tolerance import assert_transform_close, random_complex
+
+    x = random_complex(rng, (slabs, n, cols))
+    expected = _fft_columns(x, False)
+    xd = torch.from_numpy(x).cuda()
+    guard = torch.full((xd.numel() + 64,), 7.0, dtype=torch.complex64, device="cuda")
+    yd = guard[: xd.numel()].view_as(xd)
+    assert lib.spx_columns(impl, _ptr(xd), _ptr(yd), n, cols, slabs, 0, None) == SPX_OK
+    torch.cuda.synchronize()
+    assert_transform_close(yd, expected, n, axes=(-2,))
+    yd.copy_(xd)
+    assert lib.spx_columns(impl, _ptr(yd), _ptr(yd), n, cols, slabs, 0, None) == SPX_OK
+    torch.cuda.synchronize()
+    assert_transform_close(yd, expected, n, axes=(-2,))
+    assert bool((guard[xd.numel():] == 7.0).all())  # nothing past the last column
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [256, 512, 1024, 2048, 4096, 8192])
 def test_direct_pruned_r2c_at_every_row_width(lib, rng, n):
     # R2C rows of 16 .. 256 lanes at radix 8: the register combine with the staged store (16, 32
