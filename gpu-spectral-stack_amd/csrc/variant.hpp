@@ -1163,16 +1163,21 @@ struct Fused2dDriver {
         return false;
     }
 
+    // Whether the narrow-tile kernels take shapes beyond those. The radix-8 variants only: their
+    // radix-16 columns keep the two passes' accuracy; radix 4 was 2-3 % further off, and slower for
+    // few arrays (128 x 256, 64 arrays: 8.8 -> 10.5 us; 256 x 256, 128: 17.6 -> 19.7 us).
+    static constexpr bool kModesOnly = R == 8;
+
     // The shapes beyond those whose pruned transforms with w <= n2/8 take a narrow-tile kernel. One
-    // workgroup per array: 256 x 256 arrays take 10 to 12 us however few there are, against 10.6 us
-    // for 32 and 12.6 to 13.4 us for 64 in two passes (one array: two short launches), so they
-    // need 48; the smaller shapes (7 us against 10 us for one array) always win.
+    // workgroup per array: 256 x 256 arrays take 10 to 12 us however few there are, two passes 9.4
+    // to 12.5 us for 48, 10.8 to 13.5 for 56 and 11.8 to 15 for 80, so they need 56; the smaller
+    // shapes (7 us against 8.6 us for one array) always win.
     static bool modes_supports(int n1, int n2, int m1, int w, int batch)
     {
-        if constexpr (R >= 4) {
+        if constexpr (kModesOnly) {
 #define SPX_X(A, B) || (n1 == (A) && n2 == (B))
             return (false SPX_MODES_ONLY_SHAPES(SPX_X)) && m1 > 0 && w <= n2 / 8
-                   && (n1 * n2 < 65536 || batch >= 48);
+                   && (n1 * n2 < 65536 || batch >= 56);
 #undef SPX_X
         }
         return false;
@@ -1315,6 +1320,8 @@ struct Fused2dDriver {
     }
             SPX_FUSED_SHAPES(SPX_X)
 #undef SPX_X
+        }
+        if constexpr (kModesOnly) {
 #define SPX_X(A, B)                                                  \
     if (n1 == (A) && n2 == (B)) {                                    \
         launch_modes_r2c<(A), (B) / 2>(x, y, m1, w, batch, stream);  \
@@ -1533,6 +1540,8 @@ struct Fused2dDriver {
     }
             SPX_FUSED_SHAPES(SPX_X)
 #undef SPX_X
+        }
+        if constexpr (kModesOnly) {
 #define SPX_X(A, B)                                                  \
     if (n1 == (A) && n2 == (B)) {                                    \
         launch_modes_c2r<(A), (B) / 2>(x, y, m1, w, batch, stream);  \

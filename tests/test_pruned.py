@@ -129,7 +129,7 @@ def test_narrow_tile_kernels_at_their_bounds(rng, impl, n1, n2, m1, m2):
                                               (lambda n: n // 4, lambda n: n // 8 + 1)])
 def test_large_narrow_tile_kernels(rng, impl, n1, n2, m1_of, m2_of):
     m1, m2 = m1_of(n1), m2_of(n2)
-    batch = 49 if n1 * n2 == 65536 else 3  # fewer than 48 arrays of 256 x 256 take two passes
+    batch = 49 if n1 * n2 == 65536 else 3  # fewer than 56 arrays of 256 x 256 take two passes
     x = random_real(rng, (batch, n1, n2))
     y = spectral.rfft2_truncated(dev(x), m1, m2, impl=impl)
     assert_transform_close(y, ref.rfft2_truncate(x, m1, m2), n1 * n2, axes=AXES)
@@ -139,6 +139,34 @@ def test_large_narrow_tile_kernels(rng, impl, n1, n2, m1_of, m2_of):
     for few in (1, 47):  # the other side of the rule
         assert_transform_close(spectral.rfft2_truncated(dev(x[:few]), m1, m2, impl=impl),
                                ref.rfft2_truncate(x[:few], m1, m2), n1 * n2, axes=AXES)
+
+
+# 256 x 256 arrays take a narrow-tile kernel in the radix-8 variants, from 56 arrays on: below, and in
+# the other variants, an array's result does not depend on the batch it comes in, bit for bit.
+@pytest.mark.parametrize("impl, batch", [("stockham_r2", 60), ("stockham_r4", 60),
+                                         ("stockham_r4", 130), ("stockham_r8", 55),
+                                         ("stockham_r8_table", 55)])
+def test_two_pass_modes_are_the_same_in_any_batch(rng, impl, batch):
+    x = dev(random_real(rng, (batch, 256, 256)))
+    modes = dev(random_complex(rng, (batch, 32, 16)))
+    y = spectral.rfft2_truncated(x, 16, 16, impl=impl)
+    back = spectral.irfft2_from_modes(modes, (256, 256), impl=impl)
+    for few in (1, 40):
+        assert torch.equal(spectral.rfft2_truncated(x[:few], 16, 16, impl=impl), y[:few])
+        assert torch.equal(spectral.irfft2_from_modes(modes[:few], (256, 256), impl=impl),
+                           back[:few])
+
+
+@pytest.mark.parametrize("impl", ["stockham_r8", "stockham_r8_table"])
+@pytest.mark.parametrize("m1, m2", [(1, 1), (32, 16), (33, 17), (65, 31), (128, 32), (64, 33)])
+@pytest.mark.parametrize("batch", [55, 56, 57])
+def test_large_narrow_tile_kernels_at_their_first_batch(rng, impl, m1, m2, batch):
+    x = random_real(rng, (batch, 256, 256))
+    modes = random_complex(rng, (batch, 2 * m1, m2))
+    assert_transform_close(spectral.rfft2_truncated(dev(x), m1, m2, impl=impl),
+                           ref.rfft2_truncate(x, m1, m2), 65536, axes=AXES)
+    assert_transform_close(spectral.irfft2_from_modes(dev(modes), (256, 256), impl=impl),
+                           ref.irfft2_from_modes(modes, (256, 256)), 65536, axes=AXES)
 
 
 # --- the mode layout, bit for bit ------------------------------------------------------------
