@@ -17,13 +17,22 @@ constexpr int kFourStepMaxN = kStockhamMaxN * kStockhamMaxN;  // 2^24 (reference
 // C2C sizes above kStockhamMaxN that still run as one kernel per transform (the whole transform
 // in one workgroup's LDS); the multi-pass splits take over beyond.
 constexpr int kSinglePassMaxN = 16384;
-// Above that, up to kTwoPassMaxN, a column pass and a row pass that stores transposed; beyond,
-// the column pass itself runs as two. SPX_TWO_PASS_MAX_LOG2 overrides it in a variant build,
-// to measure the three-pass split at sizes the two-pass one serves.
-#ifndef SPX_TWO_PASS_MAX_LOG2
-#define SPX_TWO_PASS_MAX_LOG2 20
-#endif
+// Above that, up to kTwoPassMaxN (kSplitTwoPassMaxN in the radix-8 variants, whose 2048-point
+// columns and rows run in one pass), a column pass and a row pass that stores transposed; beyond,
+// the column pass itself runs as two. SPX_TWO_PASS_MAX_LOG2 overrides both in a variant build, to
+// measure the three-pass split at sizes the two-pass one serves.
+#ifdef SPX_TWO_PASS_MAX_LOG2
 constexpr int kTwoPassMaxN = 1 << SPX_TWO_PASS_MAX_LOG2;
+constexpr int kSplitTwoPassMaxN = kTwoPassMaxN;
+#else
+constexpr int kTwoPassMaxN = 1 << 20;
+constexpr int kSplitTwoPassMaxN = 1 << 22;
+#endif
+// The row length of the two-pass split of n points, `split`: with 2048-point rows.
+constexpr int two_pass_rows(int n, bool split)
+{
+    return n <= (1 << 18) ? 512 : n <= (1 << 21) || !split ? 1024 : 2048;
+}
 
 // reference fft.hpp:14-15, 36-39, 59-60
 using C2cFn = void (*)(const cf32* x, cf32* y, int n, int batch, Direction direction,

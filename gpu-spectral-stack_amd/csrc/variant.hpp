@@ -750,16 +750,17 @@ struct Stockham {
     // Columns of 2048 points and twiddled rows of 2048 points run in one pass (fft_split.hpp), so
     // two passes reach 2^22 points.
     static constexpr bool kSplit = R == 8 && dev::kRadix16;
+    static constexpr int kTwoPasses = kSplit ? kSplitTwoPassMaxN : kTwoPassMaxN;
 
-    // n = n1 x n2 in two passes, for kSinglePassMaxN < n <= kTwoPassMaxN (4 kTwoPassMaxN with
-    // kSplit: 2^21 = 2048 x 1024 134.7 -> 107 us over 2^24 points against the three passes, 2^22 =
-    // 2048 x 2048 143.0 -> 124.5 us, and no slower for one transform): n1-point transforms down
-    // the n2 columns of each n1 x n2 matrix (x -> work), then the twiddled n2-point rows, stored
-    // transposed (work -> y): X[k1 + n1 k2] is row k1's element k2.
+    // n = n1 x n2 in two passes, for kSinglePassMaxN < n <= kTwoPasses (with kSplit: 2^21 = 2048 x
+    // 1024 134.7 -> 107 us over 2^24 points against the three passes, 2^22 = 2048 x 2048 143.0 ->
+    // 124.5 us, and no slower for one transform): n1-point transforms down the n2 columns of each
+    // n1 x n2 matrix (x -> work), then the twiddled n2-point rows, stored transposed (work -> y):
+    // X[k1 + n1 k2] is row k1's element k2.
     static void two_pass(const cf32* x, cf32* y, int n, int batch, Direction direction,
                          hipStream_t stream, cf32* given)
     {
-        const int n2 = n <= (1 << 18) ? 512 : n <= (1 << 21) ? 1024 : 2048;
+        const int n2 = two_pass_rows(n, kSplit);
         const int n1 = n / n2;
         if (static_cast<long long>(batch) * n1 > INT_MAX
             || static_cast<long long>(batch) * n2 > INT_MAX) {
@@ -837,14 +838,14 @@ struct Stockham {
             }
             return;
         }
-        if (n <= (kSplit ? 4 * kTwoPassMaxN : kTwoPassMaxN)) {
+        if (n <= kTwoPasses) {
             two_pass(x, y, n, batch, direction, stream, work);
             return;
         }
         three_pass(x, y, n, batch, direction, stream, work);
     }
 
-    // n = n1 x 512 for kTwoPassMaxN < n <= kFourStepMaxN (n1 = 4096 .. 32768): two_pass with
+    // n = n1 x 512 for kTwoPasses < n <= kFourStepMaxN (n1 = 4096 .. 32768): two_pass with
     // its n1-point columns split again as 64 x n1b (ColumnStepIo, n1b = n1 / 64 = 64 .. 512).
     // Pass A: 64-point transforms over rows j1 n1b + j2 of each n1 x 512 matrix, twiddled by
     // w_n1^(j2 k1) (x -> y); pass B: n1b-point transforms over rows k1 n1b + j2, written to row

@@ -3,7 +3,9 @@ declared symbol, reports the registry, and rejects bad arguments with SPX_EINVAL
 reference's messages before touching the GPU. On a GPU, direct calls match the oracle."""
 
 import ctypes
+import os
 import re
+import subprocess
 from pathlib import Path
 
 import numpy as np
@@ -616,6 +618,29 @@ def test_long_columns_at_both_sides_of_the_rule(lib, rng, impl, n, cols, slabs):
     torch.cuda.synchronize()
     assert_transform_close(yd, expected, n, axes=(-2,))
     assert bool((guard[xd.numel():] == 7.0).all())  # nothing past the last column
+
+
+@pytest.mark.parametrize(("log2", "plain", "split"), [(None, 20, 22), (19, 19, 19), (22, 22, 22)])
+def test_the_two_pass_limit_follows_its_override(tmp_path, log2, plain, split):
+    # SPX_TWO_PASS_MAX_LOG2 moves the limit of every variant, and a variant without 2048-point rows
+    # never splits into them. Constants only: the host compiler's front end decides.
+    hipcc = Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "bin" / "hipcc"
+    if not hipcc.exists():
+        pytest.skip("no hipcc")
+    source = tmp_path / "limits.hip"
+    source.write_text(f"""#include "fft_api.hpp"
+static_assert(spx::kTwoPassMaxN == 1 << {plain} && spx::kSplitTwoPassMaxN == 1 << {split}, "");
+static_assert(spx::two_pass_rows(1 << 18, true) == 512, "");
+static_assert(spx::two_pass_rows(1 << 21, true) == 1024, "");
+static_assert(spx::two_pass_rows(1 << 22, true) == 2048, "");
+static_assert(spx::two_pass_rows(1 << 22, false) == 1024, "");
+""")
+    csrc = REPO / "gpu-spectral-stack_amd" / "csrc"
+    define = [] if log2 is None else [f"-DSPX_TWO_PASS_MAX_LOG2={log2}"]
+    done = subprocess.run([str(hipcc), "--offload-host-only", "-fsyntax-only", "-std=c++17",
+                           f"-I{csrc}", f"-I{REPO / 'include'}", *define, str(source)],
+                          capture_output=True, text=True, timeout=120)
+    assert done.returncode == 0, done.stderr
 
 
 @pytest.mark.gpu
