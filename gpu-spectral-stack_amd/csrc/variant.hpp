@@ -754,9 +754,10 @@ struct Stockham {
 
     // n = n1 x n2 in two passes, for kSinglePassMaxN < n <= kTwoPasses (with kSplit: 2^21 = 2048 x
     // 1024 134.7 -> 107 us over 2^24 points against the three passes, 2^22 = 2048 x 2048 143.0 ->
-    // 124.5 us, and no slower for one transform): n1-point transforms down the n2 columns of each
-    // n1 x n2 matrix (x -> work), then the twiddled n2-point rows, stored transposed (work -> y):
-    // X[k1 + n1 k2] is row k1's element k2.
+    // 124.5 us; one transform 31.9 and 46.1 -> 45.5 us, but with table twiddles 2^22 43.6 -> 45.8,
+    // which stays at three passes): n1-point transforms down the n2 columns of each n1 x n2 matrix
+    // (x -> work), then the twiddled n2-point rows, stored transposed (work -> y): X[k1 + n1 k2] is
+    // row k1's element k2.
     static void two_pass(const cf32* x, cf32* y, int n, int batch, Direction direction,
                          hipStream_t stream, cf32* given)
     {
@@ -838,7 +839,7 @@ struct Stockham {
             }
             return;
         }
-        if (n <= kTwoPasses) {
+        if (n <= kTwoPasses && !(Table && n > (1 << 21) && batch == 1)) {
             two_pass(x, y, n, batch, direction, stream, work);
             return;
         }
