@@ -1,5 +1,6 @@
 """Radio processing on this stack's FFTs: periodic windows, the spectrum of back-to-back frames,
-and FIR filtering by overlap-save, each with a selectable FFT backend. The public names, their
+and FIR filtering, by overlap-save with a selectable FFT backend or, for short real filters, as the
+convolution sum. The public names, their
 arguments and results, and the command line are the reference's (python/spectral/rf.py:1-212),
 so its callers and its RF tests run unchanged.
 
@@ -9,10 +10,12 @@ Backends (fft_impl):
 
 With a Stockham backend and a frame or block of 2 .. 16384 samples, spectrum() and fir() are one
 kernel launch each (torch.ops.spectral.rf_spectrum, rf_fir; the filter's spectrum is one more,
-rf_fir_spectrum; short real filters without a given block size are one launch, rf_fir_direct):
-frames and overlap-save blocks are read from the signal in place, with the zero
-padding decided by bounds, and the window or the filter's spectrum is applied in registers.
-Otherwise the same results are composed from tensor operations around the chosen FFT.
+rf_fir_spectrum): frames and overlap-save blocks are read from the signal in place, with the zero
+padding decided by bounds, and the window or the filter's spectrum is applied in registers. Short
+real filters without a given block size are one launch without any FFT (rf_fir_direct), the same in
+every Stockham backend, where that is less work (_summed_directly); a given block size, default_nfft
+included, runs the backend's blocks. Otherwise the same results are composed from tensor operations
+around the chosen FFT.
 
 Files are gpu-rf-pipeline's: .cf32 interleaved little-endian float32 I/Q, .f32 raw float32 taps.
 
@@ -183,7 +186,9 @@ def fir(
     x: torch.Tensor, taps: torch.Tensor, *, nfft: int | None = None, fft_impl: str = "rocfft"
 ) -> torch.Tensor:
     """y[n] = sum_k taps[k] x[n - k], zero initial state (scipy.signal.lfilter(taps, 1, x)), each
-    row of complex64 (..., n) its own signal; taps real or complex. Overlap-save: block b is the
+    row of complex64 (..., n) its own signal; taps real or complex. With a Stockham backend, short
+    real taps and no given nfft it is that sum as it stands, where it is less work than blocks.
+    Otherwise overlap-save: block b is the
     nfft samples x[b L - (M - 1) .. b L + L - 1] (zeros before the start and past the end), with
     M = len(taps) and L = nfft - M + 1; its circular convolution with the taps is exact in its
     last L outputs, which are y[b L .. b L + L - 1]."""

@@ -23,8 +23,8 @@ pytestmark = pytest.mark.gpu
 IMPLS = spectral.FFT_IMPLS
 STOCKHAM = [impl for impl in IMPLS if impl.startswith("stockham")]
 DIRECTIONS = ["forward", "inverse"]
-# 8192 and 16384: one workgroup per transform; to 2^20 a column pass and a transposing row pass;
-# beyond, the column pass runs as two (64 x n1/64 points) before the rows.
+# 8192 and 16384: one workgroup per transform; to 2^20 (2^22 in the radix-8 variants) a column pass
+# and a transposing row pass; beyond, the column pass runs as two (64 x n1/64 points) before the rows.
 MULTI_PASS = [1 << p for p in range(13, 24)]
 
 

@@ -248,8 +248,9 @@ def test_frames_take_the_many_step_path(rng):
 @pytest.mark.parametrize("pruned", [True, False], ids=["pruned", "full"])
 @pytest.mark.parametrize("n, batch", [(32, 33), (64, 5), (128, 3), (256, 7), (512, 2), (1024, 9)])
 def test_grid_steps_match_the_composed_step(rng, n, batch, pruned):
-    # Odd counts of fields leave partial workgroups; nine fields of 1024^2 run as two groups. The
-    # second state fills every mode of the layout, masked and non-Hermitian ones too. Two float32
+    # Odd counts of fields leave partial workgroups; nine fields of 1024^2 run as two groups in the
+    # full layout (7 to a group; pruned 11, and 12 fields are tested through the C ABI). The second
+    # state fills every mode of the layout, masked and non-Hermitian ones too. Two float32
     # orders of the same sums: each is 3e-7 to 5e-7 off 64 bits here.
     flow, dt = Flow(viscosity=rng.uniform(1e-3, 5e-3, batch), drag=0.1), 1e-3
     grid = GpuSolver(n, flow, dt, pruned=pruned)

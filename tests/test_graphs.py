@@ -15,6 +15,7 @@ import torch
 
 import spectral
 from oracle.tolerance import random_complex, random_real
+from spectral import rf
 from spectral.flow import Flow
 from spectral.flow.gpu import GpuSolver
 
@@ -22,7 +23,7 @@ pytestmark = pytest.mark.gpu
 
 LIB = Path(__file__).resolve().parents[1] / "gpu-spectral-stack_amd" / "python" / "spectral" \
     / "libspectral_hip.so"
-STOCKHAM_R8 = 3
+STOCKHAM_R4, STOCKHAM_R8 = 2, 3
 
 
 def replay_matches_eager(fn, inputs):
@@ -135,18 +136,73 @@ def test_navier_stokes_many_step_launch_under_capture(rng, n):
 @pytest.mark.parametrize(("n", "batch"), [(1 << 20, 2), (1 << 22, 1)])
 def test_large_c2c_without_allocation_under_capture(rng, n, batch):
     # Beyond 16384 points spx_c2c takes stream-ordered scratch; spx_c2c_noalloc, the entry point
-    # for callers that cannot allocate, uses the library's static array, so the two- and
-    # three-pass transforms can be captured.
+    # for callers that cannot allocate, uses the library's static array, so the multi-pass
+    # transforms can be captured (here two passes: the radix-8 variants', up to 2^22 points).
+    large_c2c_under_capture(rng, STOCKHAM_R8, n, batch)
+
+
+@pytest.mark.parametrize(("n", "batch"), [(1 << 21, 2), (1 << 22, 1)])
+def test_three_pass_c2c_without_allocation_under_capture(rng, n, batch):
+    large_c2c_under_capture(rng, STOCKHAM_R4, n, batch)  # three passes beyond 2^20
+
+
+def large_c2c_under_capture(rng, impl, n, batch):
     lib = ctypes.CDLL(str(LIB))
     lib.spx_last_error.restype = ctypes.c_char_p
 
     def fn(x):
         y = torch.empty_like(x)
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-        rc = lib.spx_c2c_noalloc(STOCKHAM_R8, ctypes.c_void_p(x.data_ptr()),
+        rc = lib.spx_c2c_noalloc(impl, ctypes.c_void_p(x.data_ptr()),
                                  ctypes.c_void_p(y.data_ptr()), n, batch, 0, stream)
         assert rc == 0, lib.spx_last_error().decode()
         return y
 
     inputs = [cuda(random_complex(rng, (batch, n))) for _ in range(3)]
     replay_matches_eager(fn, inputs)
+
+
+@pytest.mark.parametrize(("n", "pruned", "batch", "steps"), [(256, True, 3, 1), (256, True, 20, 3),
+                                                            (64, False, 5, 2), (512, True, 9, 2)])
+def test_navier_stokes_grid_steps_under_capture(rng, n, pruned, batch, steps):
+    # The operator itself; GpuSolver composes a captured step. Its workspace comes from torch, the
+    # kernels of a call from one stream.
+    solver = GpuSolver(n, Flow(viscosity=np.linspace(1e-3, 4e-3, batch)), 1e-3,
+                       fft_impl="stockham_r8", pruned=pruned, fused=False)
+    fields = [solver.to_spectral(cuda(random_real(rng, (batch, n, n)))) for _ in range(3)]
+    replay_matches_eager(
+        lambda w: torch.ops.spectral.ns_advance_grid(w, solver.forcing_hat, solver.nu, 0.1, 1e-3, n,
+                                                     steps, pruned),
+        fields)
+
+
+@pytest.mark.parametrize(("shape", "taps"), [((1 << 16,), 63), ((3, 5000), 129), ((4096, 64), 63),
+                                             ((1 << 16,), 200)])
+def test_filters_under_capture(rng, shape, taps):
+    # The convolution sum and, for many short rows or more taps, the blocks.
+    h = cuda(rng.standard_normal(taps).astype(np.float32))
+    inputs = [cuda(random_complex(rng, shape)) for _ in range(3)]
+    replay_matches_eager(lambda x: rf.fir(x, h, fft_impl="stockham_r8"), inputs)
+
+
+@pytest.mark.parametrize(("n1", "n2", "arrays", "m2"), [(256, 256, 60, 32), (256, 256, 60, 8),
+                                                       (128, 256, 5, 32), (256, 128, 5, 16),
+                                                       (256, 256, 5, 32)])
+def test_large_fno_modes_under_capture(rng, n1, n2, arrays, m2):
+    # Arrays in one workgroup of 512 or 1024 lanes, and few of 256^2 in two passes.
+    inputs = [cuda(random_real(rng, (arrays, n1, n2))) for _ in range(3)]
+    replay_matches_eager(
+        lambda x: spectral.irfft2_from_modes(
+            spectral.rfft2_truncated(x, m2, m2, impl="stockham_r8"), (n1, n2), impl="stockham_r8"),
+        inputs)
+
+
+@pytest.mark.parametrize(("n1", "n2", "arrays"), [(1024, 64, 40), (1024, 1024, 1), (2048, 64, 3)])
+def test_long_columns_under_capture(rng, n1, n2, arrays):
+    # Columns as register tiles, in place and out of place.
+    complex_inputs = [cuda(random_complex(rng, (arrays, n1, n2))) for _ in range(3)]
+    replay_matches_eager(lambda x: spectral.fft2(x, impl="stockham_r8"), complex_inputs)
+    inputs = [cuda(random_real(rng, (arrays, n1, n2))) for _ in range(3)]
+    replay_matches_eager(
+        lambda x: spectral.irfft2(spectral.rfft2(x, impl="stockham_r8"), n2, impl="stockham_r8"),
+        inputs)

@@ -463,3 +463,29 @@ def test_empty_recordings_filter_to_empty_ones():
         assert rf.fir(x, h, fft_impl="stockham_r8").shape == shape
     with pytest.raises(RuntimeError, match="at least one dimension"):
         rf.fir(torch.zeros((), dtype=torch.complex64, device="cuda"), h, fft_impl="stockham_r8")
+
+
+# fir() with short real taps and no block size is the convolution sum in every Stockham variant; a
+# given block size, the default one too, runs that variant's blocks.
+@pytest.mark.gpu
+@pytest.mark.parametrize("fft_impl", ONE_LAUNCH)
+@pytest.mark.parametrize(("n", "m"), [(1000, 1), (5, 63), (63, 63), (1000, 63), (4097, 64),
+                                      (50_000, 129)])
+def test_default_blocks_of_every_variant(rng, n, m, fft_impl):
+    x, taps = random_complex(rng, n), random_real(rng, m)
+    y = rf.fir(on_gpu(x), on_gpu(taps), nfft=rf.default_nfft(m), fft_impl=fft_impl)
+    assert rel_l2(y, filtered(x, taps)) < 2e-5
+    summed = rf.fir(on_gpu(x), on_gpu(taps), fft_impl=fft_impl)
+    assert torch.equal(summed, rf.fir(on_gpu(x), on_gpu(taps), fft_impl="stockham_r2"))
+    assert rel_l2(summed, filtered(x, taps)) < 2e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["bpsk", "qpsk"])
+def test_recordings_decode_through_the_default_blocks(name):
+    samples, meta = recording(name)
+    taps = rf.read_f32(GOLDEN_RF / meta["pulse"])
+    y = rf.fir(on_gpu(samples), on_gpu(taps), nfft=rf.default_nfft(len(taps)),
+               fft_impl="stockham_r8")
+    decided, sent = matched_filter_decisions(name, y.cpu().numpy())
+    assert np.array_equal(decided, sent)
