@@ -367,8 +367,9 @@ __device__ __forceinline__ void update_columns(cf32 (&v)[G::PC::E], cf32* s, con
         const int i = row_of(e);
         const int r = state_row<G>(i);
         const float ky = ky_of<G>(i);
-        const bool kept = kx <= kmax && fabsf(ky) <= kmax;
-        const cf32 F = csub(forcing[e], kept ? v[e] : czero());
+        // A product, so that a field that has overflowed spreads to every mode, as N_hat * mask does.
+        const float mask = kx <= kmax && fabsf(ky) <= kmax ? 1.0f : 0.0f;
+        const cf32 F = csub(forcing[e], cscale(v[e], mask));
         const float linear = -nu_f * (kx * kx + ky * ky) - a.drag;
         const float ex = 1.0f + 0.5f * a.dt * linear;
         const float im = reciprocal(1.0f - 0.5f * a.dt * linear);

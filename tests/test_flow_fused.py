@@ -466,3 +466,23 @@ def test_a_subclass_may_build_advance_on_step(rng, n, pruned):
     plain = GpuSolver(n, Flow(viscosity=2e-3), 1e-3, pruned=pruned)
     expected = plain.step(plain.step(plain.step(w)))
     assert torch.equal(solver.advance(w, 3), expected) and solver.count == 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pruned", [True, False], ids=["pruned", "full"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_grid_steps_spread_what_the_composed_step_spreads(rng, bad, pruned):
+    # A field with a NaN or an infinity is lost in every mode, the dealiased ones too; its
+    # neighbours step on.
+    n = 32
+    solver = GpuSolver(n, Flow(viscosity=2e-3), 1e-3, pruned=pruned)
+    composed = GpuSolver(n, Flow(viscosity=2e-3), 1e-3, pruned=pruned, fused=False)
+    clean = random_state(rng, n, (3,), composed)
+    w = clean.clone()
+    w[1, 3, 2] = complex(bad, 0.5)
+    assert solver._takes_grid_steps(w)
+    got, expected = solver.step(w), composed.step(w)
+    assert torch.isnan(torch.view_as_real(expected[1])).any(-1).all()
+    assert torch.isnan(torch.view_as_real(got[1])).any(-1).all()
+    for field in (0, 2):
+        assert relative(got[field], expected[field]) < 3e-6  # two float32 orders
