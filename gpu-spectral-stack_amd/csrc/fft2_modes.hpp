@@ -19,9 +19,9 @@
 //            prepare), inverse row transform, the real rows stored.
 //
 // Arrays of 2^15 and 2^16 points (128 x 256, 256 x 128, 256 x 256), whose half spectra fit no
-// workgroup, take the same kernels with 512 or 1024 lanes, in place of a row pass and a column pass
-// through HBM. 256 x 256 x 256, 32 modes, forward / inverse: 28.5 / 29.3 us in two passes, 18.0 /
-// 17.8 us here; 512 arrays 43.7 / 50.1 -> 34.4 / 32.7 us. With one array per compute unit the
+// workgroup, take the same kernels with 512 or 1024 lanes in the radix-8 variants, in place of a row
+// pass and a column pass through HBM. 256 x 256 x 256, 32 modes, forward / inverse: 28.4 / 29.7 us in
+// two passes, 16.9 / 17.9 us here; 512 arrays 43.7 / 50.1 -> 34.4 / 32.7 us. With one array per compute unit the
 // row transforms' instructions (9 us per array) and the loads at the HBM rate (11 us for 256
 // arrays) overlap pass by pass; the last pass and the columns stay outside.
 //

@@ -6,8 +6,9 @@
 // of 2048 points 139 KB, where complex exchanges hold 8 and 4. Every global access is then a run of
 // 16 values, a whole 128-byte line: tiles of 8 columns read half a line per row, whose other half
 // belongs to another workgroup. A column pass of 1024-point columns over 2^24 points went from
-// 69.9 to 58.7 us (4.6 TB/s, what a copy in that pattern reaches). Rows of 1024 points keep 8 to a
-// workgroup (46.6 us; 16 split rows 47.5 us, and 9.2 against 11.8 us for one 2^20 transform).
+// 69.9 to 58.8 us (4.6 TB/s, what a copy in that pattern reaches; in place, behind a row pass, 44.5).
+// Rows of 1024 points keep 8 to a workgroup (46.6 us; 16 split rows 47.5 us, and 9.2 against 11.8 us
+// for one 2^20 transform).
 
 #include "stockham.hpp"
 

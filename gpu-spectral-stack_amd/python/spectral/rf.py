@@ -1,8 +1,7 @@
 """Radio processing on this stack's FFTs: periodic windows, the spectrum of back-to-back frames,
 and FIR filtering, by overlap-save with a selectable FFT backend or, for short real filters, as the
-convolution sum. The public names, their
-arguments and results, and the command line are the reference's (python/spectral/rf.py:1-212),
-so its callers and its RF tests run unchanged.
+convolution sum. The public names, their arguments and results, and the command line are the
+reference's (python/spectral/rf.py:1-212), so its callers and its RF tests run unchanged.
 
 Backends (fft_impl):
     "rocfft" / "cufft"   torch.fft (rocFFT on ROCm); "cufft" is the reference's name for it

@@ -176,12 +176,13 @@ int spx_ns_steps(const void* w_in, void* w_out, void* work, const void* forcing_
                  const float* nu, int nu_stride, float drag, float dt, int n, int batch,
                  int steps, hipStream_t stream);
 
-/* spx_ns_grid_steps: the same steps for the grids and layouts without a one-workgroup kernel, two
- * launches per stage and one more each for a call's start and end: n a power of two from 32 to 1024 (spx_ns_grid_supports), the pruned layout
- * above or (pruned = 0) the rfft2 layout, n x (n/2 + 1) values per field. `steps` >= 1 steps of
- * w_in into w_out, which are the same array or do not overlap; `work` holds
- * spx_ns_grid_workspace complex values and overlaps no other array. forcing_hat: one field's
- * values in the layout, shared by all fields. Replaces python/spectral/flow/gpu.py:115-142. */
+/* spx_ns_grid_steps: the same steps for the grids and layouts without a one-workgroup kernel, in
+ * 4 * steps + 1 launches per group of fields (as many as keep the derived spectra within 128 MB): n a
+ * power of two from 32 to 1024 (spx_ns_grid_supports), the pruned layout above or (pruned = 0) the
+ * rfft2 layout, n x (n/2 + 1) values per field. `steps` >= 1 steps of w_in into w_out, which are the
+ * same array or do not overlap; `work` holds spx_ns_grid_workspace complex values (never
+ * fewer for a larger batch) and overlaps no other array. forcing_hat: one field's values in the
+ * layout, shared by all fields. Replaces python/spectral/flow/gpu.py:115-142. */
 int spx_ns_grid_supports(int n);
 int spx_ns_grid_workspace(int n, int pruned, int batch, size_t* count);
 int spx_ns_grid_steps(const void* w_in, void* w_out, void* work, const void* forcing_hat,
@@ -203,7 +204,8 @@ int spx_ns_grid_steps(const void* w_in, void* w_out, void* work, const void* for
  *                    1 <= count <= nfft, in one launch; it replaces rf.py:145-147 (zeros, a copy
  *                    of the converted taps, fft).
  *   spx_rf_fir_direct  the same y from the taps themselves, 1 <= count <= spx_rf_fir_direct_taps()
- *                    float32 values: the convolution sum on the matrix cores, no blocks. */
+ *                    float32 values: the convolution sum on the matrix cores, no blocks. It runs
+ *                    whole steps of 1024 outputs per row: for long rows. */
 int spx_rf_fir_direct_taps(void);
 int spx_rf_fir_direct(const void* x, const float* taps, void* y, long long n, int count,
                       long long rows, hipStream_t stream);
