@@ -23,9 +23,9 @@
 //                      with F = f_hat - mask N_hat, e = 1 + dt/2 L, i = 1 / (1 - dt/2 L),
 //                      L = -nu |k|^2 - alpha.
 // A call's first stage takes its columns from ns_columns_kernel and its last one ends in
-// ns_update_kernel: 4 steps + 1 launches per group of fields. The derived spectra (4 n pitch values per field) are the one large
-// intermediate. Normalization: inverse 1 / n^2, forward none, as numpy. The imaginary parts of a
-// row's zero and n/2 frequencies are dropped, as numpy's irfft drops them.
+// ns_update_kernel: 4 steps + 1 launches per group of fields. The derived spectra (4 n pitch values
+// per field) are the one large intermediate. Normalization: inverse 1 / n^2, forward none, as numpy.
+// The imaginary parts of a row's zero and n/2 frequencies are dropped, as numpy's irfft drops them.
 //
 // Measured on MI355X (256^2 pruned, 48 fields, six steps and a frame): 434 us with the update and
 // the columns apart (10.3 and 12.8 us; rows 13.0 us), 349 us as here (rows 13.0, update and

@@ -906,11 +906,11 @@ struct Stockham {
     }
 
     // Columns of n = 2048 (where not split_columns) or 4096 points as two passes of 64 x (n / 64) (a
-    // four-step split of the column axis): a single pass would stage only 4 or 2 columns per workgroup, reading
-    // runs of 32 or 16 bytes; each of these passes stages 32 columns of 64 points (256-byte
-    // runs). Pass A runs
-    // the 64-point transforms over rows j1 (n/64) + j2 and twiddles them (x -> work); pass B runs
-    // the (n/64)-point transforms over rows k1 (n/64) + j2 and writes row k1 + 64 k2 (work -> y).
+    // four-step split of the column axis): a single pass would stage only 4 or 2 columns per
+    // workgroup, reading runs of 32 or 16 bytes; each of these passes stages 32 columns of 64 points
+    // (256-byte runs). Pass A runs the 64-point transforms over rows j1 (n/64) + j2 and twiddles them
+    // (x -> work); pass B runs the (n/64)-point transforms over rows k1 (n/64) + j2 and writes row
+    // k1 + 64 k2 (work -> y).
     static void long_columns(const cf32* x, cf32* y, int n, int cols, int slabs,
                              Direction direction, hipStream_t stream, bool stream_out)
     {
